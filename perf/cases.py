@@ -95,11 +95,6 @@ def draw(rng):
 
 # -------------------------------------------------------------------------------------- their inputs
 
-def _coord_grid(n, start, stop, bias):
-    b = (stop - start) / math.expm1(bias)
-    return b * np.expm1(bias * np.arange(n) / (n - 1.0)) + start
-
-
 def _dressing(r, n):
     """A smooth dressing function Z in (0.5, 1.5): a random sum of four waves through tanh."""
     i = np.arange(n)
