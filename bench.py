@@ -42,14 +42,18 @@ GRAPH_SETS = 10  # call sets per hipGraph launch
 # loops of se_kernel<MODE, BLOCK, UNROLL>, counted from the gfx950 assembly of
 # csrc/integrals.hip by `python -m diffrg_amd.isa_count`: "pairs" when a lane owns two angular
 # pairs (na^2 >= 2 BLOCK), "pairs2" the same loop taking two radial nodes per step (the mixed
-# path's unroll 2, SEBatch.unroll), "single" when a lane owns one pair and two radial nodes per
+# unroll 2, SEBatch.unroll(MIXED), which the seeded FP64 form shares), "single" when a lane owns one pair and two radial nodes per
 # iteration.  tests/test_isa_counts.py checks these figures against the current source.
 # Keyed by the integrand form (SEBatch.variants): 0 FP64, 1 mixed, 2 mixed on an integral that
 # admits the narrow exponent rounding.
-SE_OPS = {0: {"pairs": (223.5, 203.0), "single": (223.5, 205.0)},
+# FP64 runs the seeded form ("seeded") on integrals whose coordinates and tables admit it, as those of
+# every workload here do, and the library-call form 0 on the others.
+SE_OPS = {0: {"pairs": (223.5, 203.0), "single": (223.5, 205.5)},
+          "seeded": {"pairs": (63.5, 50.0), "pairs2": (63.25, 49.0), "single": (63.5, 52.0)},
           1: {"pairs": (46.0, 44.0), "pairs2": (46.0, 43.5), "single": (46.0, 46.0)},
           2: {"pairs": (46.0, 42.0), "pairs2": (46.0, 41.5), "single": (46.0, 44.0)}}
-SE_OPS_BLOCK = {}  # (mode, block, loop) whose schedule differs from the others
+# (form, block, loop) whose schedule differs from the others
+SE_OPS_BLOCK = {(0, 1024, "single"): (223.5, 205.0)}
 
 
 BASELINE_NOTES = "BASELINE.md"
@@ -88,7 +92,12 @@ def se_variant(b, mode):
     """The integrand form of a batch whose integrals all use the same one."""
     v = np.unique(b.variants(mode))
     assert len(v) == 1, v
-    return int(v[0])
+    return se_form(v[0])
+
+
+def se_form(variant):
+    """Key of SE_OPS for SEBatch.variants' value on the integrals of these workloads."""
+    return "seeded" if variant == 0 else int(variant)
 
 
 def valu_issue_frac(valu_per_eval, evals, seconds):
@@ -290,7 +299,7 @@ def selfenergy(D, qp, args):
                 err = max(err, rel_err(o.to_host(), ref))
         ms = min(ms_eager, ms_graph)
         res[name] = {"ms": ms, "ms_eager": ms_eager, "ms_graph": ms_graph, "ms_streams": ms_streams, "shape": shape,
-                     "err": err, "launch": "hipGraph" if ms_graph < ms_eager else "eager", "unroll": b.unroll(mode)}
+                     "err": err, "launch": "hipGraph" if ms_graph < ms_eager else "eager", "unroll": b.unroll(D.MIXED)}
         log(f"selfenergy {name}: eager {ms_eager * 1e3:.1f} us, graph {ms_graph * 1e3:.1f} us, "
             f"{N_STREAMS} streams {ms_streams * 1e3:.1f} us per call set, "
             f"err {err:.2e}, shape {shape}")
@@ -307,7 +316,7 @@ def selfenergy(D, qp, args):
     for mode, name in ((D.FP64, "fp64"), (D.MIXED, "mixed")):
         shape = bb.autotune(mode, reps=3)
         ms, _ = time_steps(D, lambda: bb.run(outb, mode), max(1, args.steps // BATCH), max(1, args.warmup // BATCH))
-        va = se_ops(se_variant(bb, mode), c["na"], shape["block"], bb.unroll(mode))[1]
+        va = se_ops(se_variant(bb, mode), c["na"], shape["block"], bb.unroll(D.MIXED))[1]
         fl = FROZEN["C1_selfenergy"][name]["flop"]
         res[name][f"batched_x{BATCH}"] = {
             "integrals_per_s": nb / (ms * 1e-3), "us_per_launch": ms * 1e3, "shape": shape,
@@ -444,8 +453,8 @@ def uneven(D, qp, args):
         r[name] = {"integrals_per_s": n / (ms * 1e-3), "evals_per_s": b.evals / (ms * 1e-3), "ms_per_batch": ms,
                    "max_rel_err": rel_err(out.to_host(), ref), "shape": shape,
                    "roofline_frac": wt["flop"] * b.evals / (ms * 1e-3) / PEAK_FP64_VALU, "ceiling": ceiling(wt),
-                   "valu_issue_frac": sum(int(q) * int(a) ** 2 * se_ops(int(v), int(a), shape["block"],
-                                                                          b.unroll(mode))[1]
+                   "valu_issue_frac": sum(int(q) * int(a) ** 2 * se_ops(se_form(v), int(a), shape["block"],
+                                                                          b.unroll(D.MIXED))[1]
                                           for q, a, v in zip(c["nq"], c["na"], b.variants(mode)))
                                       / 64 / (ms * 1e-3)
                                       / PEAK_VALU_WAVE_INSTR}

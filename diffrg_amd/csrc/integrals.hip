@@ -211,7 +211,8 @@ namespace
     int integral, q0, nqt, slot;
     int na, l2na, xq_off, xa_off; // node offsets: x at off, w at off + order
     int nq, tab_off, ntab, first_slot;
-    int n_slots, narrow, pad1, pad2; // narrow: the mixed path may use se_G_mixed<true>
+    int n_slots, narrow, seeded, pad; // narrow: the mixed path may use se_G_mixed<true>
+                                      // seeded: the FP64 path may use SESeeded
   };
 
   struct SECellZ {
@@ -230,7 +231,7 @@ namespace
     const double *nodes;
     const double *tab64;  // FP64 tables
     const SECellY *tabA;  // mixed-path cell data: (y_i^2, 1/(b + y_i - c), y_i)
-    const SECellZ *tabB;  // mixed-path cell data: (Z_i, Z_{i+1} - Z_i)
+    const SECellZ *tabB;  // cell data of the mixed and seeded FP64 paths: (Z_i, Z_{i+1} - Z_i)
     double x_extent, k, pref; // pref = 2pi/(2pi)^4
     double *partials;   // one line per tile (dev::kSlotStride)
     unsigned *counters; // one line per integral (dev::kCounterStride)
@@ -244,6 +245,9 @@ namespace
     int shared, tiles_per_int;
     const double *p_ext;
     SETile proto;
+    // dev::log_tab entries (1/c_j, -log(1/c_j)) of the seeded FP64 path, then 2^(j/64), j = 0..63
+    // (last: the mixed kernels, which do not read it, keep their argument loads)
+    const double2 *logtab;
   };
 
   // Blocks are dispatched to the eight XCDs in turn (block b to XCD b mod 8).  With xcd_map, the
@@ -268,6 +272,37 @@ namespace
     const double Z = dev::lerp_log_f64(tab, ntab, c, inv_b, scale, y);
     return 1.0 / (Z * pq2 + k2 * exp(-(pq2 / k2)));
   }
+
+  // G(|p-q|) in FP64 without library sequences.  VALU issue bounds the FP64 path, and ocml's log1p,
+  // exp and sqrt and the compiler's division take 203 VALU instructions per evaluation; the
+  // hardware's FP64 reciprocal and reciprocal-square-root estimates with one third-order step, and
+  // table-driven log and exp (device.hh), take 50 to the same accuracy (against long double, over
+  // 1,300 integrals of all orders and table sizes: largest error 6.1e-16, 6.0e-16 before).  The cell
+  // is floor of the FP64 index as in the reference, so the interpolation's kinks stay where they
+  // are.  1,023 uneven integrals (87M evaluations): 502 -> 151 us; 64 integrals of {64, 32, 32}
+  // nodes: 31.9 -> 12.0 us.  For integrals with a coordinate map of bias >= 2 whose log argument stays
+  // positive, finite table values and |64 t| < 2^30 (rule in dfrg_se_batch_create); the others keep
+  // se_G_fp64.
+  struct SESeeded {
+    const SECellZ *tabB;
+    const double2 *lg;    // (1/c_j, -scale log(1/c_j))
+    const double *exp2k;  // k^2 2^(j/64)
+    double w0, inv_b, scale, scale_ln2, last, ek64; // w0 = 1 - c/b, last = n - 1
+    // Z at y on the clamped log coordinate
+    __device__ __forceinline__ double Z(double y) const
+    {
+      const double idx = fmax(0.0, fmin(dev::log_tab(fma(y, inv_b, w0), lg, scale, scale_ln2), last));
+      const double fl = floor(idx);
+      const SECellZ cz = tabB[(int)fl];
+      return fma(idx - fl, cz.dz, cz.z);
+    }
+    // k^2 exp(-s/k^2)
+    __device__ __forceinline__ double R(double s) const { return dev::exp2_tab(s, ek64, exp2k); }
+    __device__ __forceinline__ double operator()(double s) const
+    {
+      return dev::rcp_f64(fma(Z(dev::sqrt_f64(s)), s, R(s)));
+    }
+  };
 
   struct SEMixed {
     const SECellY *tabA;
@@ -406,14 +441,19 @@ namespace
     return acc;
   }
 
+  // MODE DFRG_FP64 holds both FP64 forms (per tile); kSeededOnly, for batches whose integrals all
+  // admit the seeded form, only that one, with its register budget (the library sequences of the
+  // general form need 168 VGPRs).
+  constexpr int kSeededOnly = 2;
   template <int MODE, int BLOCK, int UNROLL> __global__ __launch_bounds__(BLOCK) void se_kernel(SEArgs A)
   {
-    constexpr bool F64 = MODE == DFRG_FP64;
-    __shared__ double s_tab64[F64 ? kMaxTab : 1];
+    constexpr bool F64 = MODE != DFRG_MIXED, GENERAL = MODE == DFRG_FP64;
+    __shared__ double s_tab64[GENERAL ? kMaxTab : 1];
     __shared__ SECellY s_tabA[F64 ? 1 : kMaxTab];
-    __shared__ SECellZ s_tabB[F64 ? 1 : kMaxTab];
-    __shared__ double s_exp2[F64 ? 1 : 64];  // 2^(j/64)
-    __shared__ double s_exp2k[F64 ? 1 : 64]; // k^2 2^(j/64)
+    __shared__ SECellZ s_tabB[kMaxTab];
+    __shared__ double2 s_log[F64 ? dev::kLogTab : 1];
+    __shared__ double s_exp2[F64 ? 1 : 64]; // 2^(j/64)
+    __shared__ double s_exp2k[64];          // k^2 2^(j/64)
     __shared__ double2 s_ang[kMaxAng]; // (cos1, 2 w1 sqrt(1 - cos1^2))
     __shared__ double s_w2[kMaxAng];   // 2 w2
     __shared__ double s_qs[kMaxQ], s_qc[kMaxQ], s_qt[kMaxQ];
@@ -428,6 +468,9 @@ namespace
         s_exp2[j] = exp2(j * (1.0 / 64.0));
         s_exp2k[j] = A.k * A.k * s_exp2[j];
       }
+    } else if ((int)threadIdx.x >= BLOCK - 64) {
+      const int j = (int)threadIdx.x - (BLOCK - 64);
+      s_exp2k[j] = A.k * A.k * ((const double *)(A.logtab + dev::kLogTab))[j];
     }
     const double k = A.k, k2 = k * k;
     int cur = -1; // integral whose table and angular terms are in LDS (block-uniform)
@@ -456,7 +499,13 @@ namespace
       // one round of independent loads: table and angular terms (when the integral changes) and
       // the radial nodes of this tile
       if (i != cur) {
-        if (F64) {
+        if (F64 && (!GENERAL || T.seeded)) {
+          for (int j = threadIdx.x; j < T.ntab; j += BLOCK) s_tabB[j] = A.tabB[T.tab_off + j];
+          for (int j = threadIdx.x; j < dev::kLogTab; j += BLOCK) {
+            const double2 l = A.logtab[j];
+            s_log[j] = make_double2(l.x, T.scale * l.y);
+          }
+        } else if (GENERAL) {
           for (int j = threadIdx.x; j < T.ntab; j += BLOCK) s_tab64[j] = A.tab64[T.tab_off + j];
         } else {
           for (int j = threadIdx.x; j < T.ntab; j += BLOCK) {
@@ -481,15 +530,31 @@ namespace
         s_qw[j] = make_double2(q, xq[T.nq + T.q0 + j] * A.x_extent);
       }
       __syncthreads();
-      // q-only factor from the staged table: el * w_q x_ext * RBdot(q) G(q)^2.  Plain mode: the
-      // reference's FP64 expression tree.  Mixed mode: FP64-accurate seeded forms (FP32 hardware
+      SESeeded S; // the seeded FP64 form's constants (unused otherwise)
+      if (F64) {
+        S.tabB = s_tabB;
+        S.lg = s_log;
+        S.exp2k = s_exp2k;
+        S.w0 = fma(-T.c, T.inv_b, 1.0);
+        S.inv_b = T.inv_b;
+        S.scale = T.scale;
+        S.scale_ln2 = T.scale * kLn2;
+        S.last = (double)(T.ntab - 1);
+        S.ek64 = -64.0 * kLog2e / k2;
+      }
+      // q-only factor from the staged table: el * w_q x_ext * RBdot(q) G(q)^2.  Plain mode: the seeded
+      // FP64 form or the reference's FP64 expression tree.  Mixed mode: FP64-accurate seeded forms (FP32 hardware
       // log2 / reciprocal seeds with FP64 Newton steps, table exp), since this factor multiplies
       // every evaluation of its radial node and its error would not average out.
       for (int j = threadIdx.x; j < T.nqt; j += BLOCK) {
         const double2 qw = s_qw[j];
         const double q = qw.x, q2 = q * q;
         double qt;
-        if (F64) {
+        if (F64 && (!GENERAL || T.seeded)) {
+          const double R = S.R(q2), Gq = dev::rcp_f64(fma(S.Z(q), q2, R));
+          const double el = A.pref * (q2 * 0.5 * k2);
+          qt = el * qw.y * (2.0 * R * (1.0 + q2 / k2)) * Gq * Gq;
+        } else if (GENERAL) {
           const double xr = q2 / k2;
           const double ex = exp(-xr);
           const double Zq = dev::lerp_log_f64(s_tab64, T.ntab, T.c, T.inv_b, T.scale, q);
@@ -514,9 +579,11 @@ namespace
       __syncthreads();
 
       double acc;
-      if (F64) {
+      if (F64 && (!GENERAL || T.seeded)) { // tile-uniform
+        acc = se_tile_sum<BLOCK, UNROLL>(S, T.na, T.l2na, T.nqt, s_ang, s_w2, s_qs, s_qc, s_qt);
+      } else if (GENERAL) {
         const auto g = [&](double pq2) { return se_G_fp64(s_tab64, T.ntab, T.c, T.inv_b, T.scale, k2, pq2); };
-        acc = se_tile_sum<BLOCK, UNROLL>(g, T.na, T.l2na, T.nqt, s_ang, s_w2, s_qs, s_qc, s_qt);
+        acc = se_tile_sum<BLOCK, 1>(g, T.na, T.l2na, T.nqt, s_ang, s_w2, s_qs, s_qc, s_qt);
       } else {
         SEMixed m;
         m.tabA = s_tabA;
@@ -602,6 +669,7 @@ struct dfrg_se_batch {
   double *d_nodes = nullptr, *d_tab64 = nullptr, *d_p = nullptr;
   SECellY *d_tabA = nullptr;
   SECellZ *d_tabB = nullptr;
+  double2 *d_log = nullptr; // SEArgs::logtab
   SETile *d_tiles = nullptr;
   double *d_partials = nullptr;
   unsigned *d_counters = nullptr, *d_queue = nullptr;
@@ -609,6 +677,8 @@ struct dfrg_se_batch {
   // shape
   int block = 256, tile_evals = 8192, grid = 0, n_tiles = 0;
   std::vector<int> narrow; // per integral: the mixed path may use se_G_mixed<true>
+  std::vector<int> seeded; // per integral: the FP64 path may use SESeeded
+  bool all_seeded = false;
   int uniform_tiles = 0;    // every tile has the same evaluation count
   int shared_layout = 0;    // every tile record follows from proto and its index (SEArgs::shared)
   int tiles_per_int = 0;
@@ -661,6 +731,7 @@ namespace
         t.first_slot = first;
         t.n_slots = cnt;
         t.narrow = b->narrow[i];
+        t.seeded = b->seeded[i];
         tiles.push_back(t);
       }
     }
@@ -727,12 +798,14 @@ namespace
     a.tiles_per_int = b->tiles_per_int > 0 ? b->tiles_per_int : 1;
     a.p_ext = b->d_p;
     a.proto = b->proto;
+    a.logtab = b->d_log;
     return a;
   }
 
-  // Radial unroll of the mixed paired loop: 2 when the launch puts at most 16 waves on a CU (4 per
+  // Radial unroll of the mixed and seeded FP64 paired loops: 2 when the launch puts at most 16 waves on a CU (4 per
   // SIMD), where four independent evaluation chains per lane hide more latency than two; 1 for
-  // fuller launches, which hide it with waves.  Results do not depend on it.
+  // fuller launches, which hide it with waves.  Results do not depend on it.  Seeded FP64 form, 64
+  // integrals of {64, 32, 32} nodes: 12.3 us with 1, 12.0 with 2.
   int se_unroll(const dfrg_se_batch *b)
   {
     const long long cus = context().cu_count > 0 ? context().cu_count : 256;
@@ -755,7 +828,9 @@ namespace
       a.queue = scr->queue;
     }
     const int grid = b->grid > 0 ? std::min(b->grid, b->n_tiles) : b->n_tiles;
-    hipError_t e = mode == DFRG_FP64    ? launch_se<DFRG_FP64, 1>(b->block, grid, s, a)
+    hipError_t e = mode == DFRG_FP64
+                       ? (b->all_seeded ? (se_unroll(b) == 2 ? launch_se<kSeededOnly, 2>(b->block, grid, s, a) : launch_se<kSeededOnly, 1>(b->block, grid, s, a))
+                                        : launch_se<DFRG_FP64, 1>(b->block, grid, s, a))
                    : se_unroll(b) == 2 ? launch_se<DFRG_MIXED, 2>(b->block, grid, s, a)
                                        : launch_se<DFRG_MIXED, 1>(b->block, grid, s, a);
     if (e != hipSuccess) {
@@ -945,6 +1020,29 @@ int dfrg_se_batch_create(dfrg_se_batch **out, dfrg_qp *qp, int n_int, const doub
       b->narrow[i] = start[i] >= 1e-30 && pq * pq * 64.0 * kLog2e / (k * k) < 1073741824.0;
     }
   }
+  // the seeded FP64 form, per integral: the narrow form's conditions (which bound |p - q|^2 and the
+  // exponent), a coordinate map of bias >= 2 (log_tab is exact to an absolute rounding, which the index
+  // multiplies by (n - 1)/bias: at bias 0.01 the results were off by 1e-12, at 2 the index is as
+  // exact at the table's end as log1p's) whose log argument 1 + (y - start)/b stays positive down to
+  // y = 0, k^2 far from the ends of the FP64 range, and finite cells (0 times an infinite slope is
+  // NaN where the reference's two-sided form gives the node)
+  b->seeded.resize(n_int);
+  for (int i = 0; i < n_int; ++i) {
+    const double bb = (stop[i] - start[i]) / std::expm1(bias[i]);
+    bool ok = b->narrow[i] && bias[i] >= 2.0 && std::isfinite(bb) && 1.0 - start[i] / bb >= 0x1p-10 &&
+              (std::fabs(p[i]) + k * std::sqrt(x_extent)) / bb < 0x1p100 && k * k > 0x1p-200 && k * k < 0x1p200;
+    for (int j = 0; ok && j < tab_n[i]; ++j) ok = std::fabs(tables[tab_off[i] + j]) < 0x1p1000;
+    b->seeded[i] = ok;
+  }
+  b->all_seeded = std::all_of(b->seeded.begin(), b->seeded.end(), [](int v) { return v != 0; });
+  // log and exp tables of the seeded form
+  std::vector<double> logtab(2 * dev::kLogTab + 64);
+  for (int j = 0; j < dev::kLogTab; ++j) {
+    const double inv = (double)(1.0L / (0.5L + (j + 0.5L) / (2 * dev::kLogTab)));
+    logtab[2 * j] = inv;
+    logtab[2 * j + 1] = (double)-std::log((long double)inv);
+  }
+  for (int j = 0; j < 64; ++j) logtab[2 * dev::kLogTab + j] = (double)std::exp2((long double)j / 64.0L);
   // cell data of the mixed path (coordinates.hh:141-196 LogarithmicCoordinates1D): node
   // y_i = b expm1(a i/(n-1)) + c, 1/(b + y_i - c), Z_i and Z_{i+1} - Z_i
   std::vector<SECellY> tabA(tables_len);
@@ -973,14 +1071,23 @@ int dfrg_se_batch_create(dfrg_se_batch **out, dfrg_qp *qp, int n_int, const doub
     }                                                                                                          \
   } while (0)
   // the inputs and the ticket counters in one allocation, so a block's first loads and its
-  // cross-block finish stay within a few pages
+  // cross-block finish stay within a few pages, staged on the host and uploaded with one copy
   {
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     const size_t o_tab64 = up(sizeof(double) * nodes.size()), o_tabA = o_tab64 + up(sizeof(double) * tables_len);
     const size_t o_tabB = o_tabA + up(sizeof(SECellY) * tables_len), o_p = o_tabB + up(sizeof(SECellZ) * tables_len);
     const size_t o_cnt = o_p + up(sizeof(double) * n_int);
     const size_t o_queue = o_cnt + up(sizeof(unsigned) * dev::kCounterStride * n_int);
-    DFRG_HIP_B(hipMalloc(&b->d_inputs, o_queue + up(sizeof(unsigned) * 2 * dev::kCounterStride)));
+    const size_t o_log = o_queue + up(sizeof(unsigned) * 2 * dev::kCounterStride);
+    std::vector<char> host(o_log + sizeof(double) * logtab.size()); // counters and queue start at zero
+    std::memcpy(&host[0], nodes.data(), sizeof(double) * nodes.size());
+    std::memcpy(&host[o_tab64], tables, sizeof(double) * tables_len);
+    std::memcpy(&host[o_tabA], tabA.data(), sizeof(SECellY) * tables_len);
+    std::memcpy(&host[o_tabB], tabB.data(), sizeof(SECellZ) * tables_len);
+    std::memcpy(&host[o_p], p, sizeof(double) * n_int);
+    std::memcpy(&host[o_log], logtab.data(), sizeof(double) * logtab.size());
+    DFRG_HIP_B(hipMalloc(&b->d_inputs, host.size()));
+    DFRG_HIP_B(hipMemcpy(b->d_inputs, host.data(), host.size(), hipMemcpyHostToDevice));
     char *base = (char *)b->d_inputs;
     b->d_nodes = (double *)base;
     b->d_tab64 = (double *)(base + o_tab64);
@@ -989,14 +1096,8 @@ int dfrg_se_batch_create(dfrg_se_batch **out, dfrg_qp *qp, int n_int, const doub
     b->d_p = (double *)(base + o_p);
     b->d_counters = (unsigned *)(base + o_cnt);
     b->d_queue = (unsigned *)(base + o_queue);
+    b->d_log = (double2 *)(base + o_log);
   }
-  DFRG_HIP_B(hipMemcpy(b->d_nodes, nodes.data(), sizeof(double) * nodes.size(), hipMemcpyHostToDevice));
-  DFRG_HIP_B(hipMemcpy(b->d_tab64, tables, sizeof(double) * tables_len, hipMemcpyHostToDevice));
-  DFRG_HIP_B(hipMemcpy(b->d_tabA, tabA.data(), sizeof(SECellY) * tables_len, hipMemcpyHostToDevice));
-  DFRG_HIP_B(hipMemcpy(b->d_tabB, tabB.data(), sizeof(SECellZ) * tables_len, hipMemcpyHostToDevice));
-  DFRG_HIP_B(hipMemcpy(b->d_p, p, sizeof(double) * n_int, hipMemcpyHostToDevice));
-  DFRG_HIP_B(hipMemset(b->d_counters, 0, sizeof(unsigned) * dev::kCounterStride * n_int));
-  DFRG_HIP_B(hipMemset(b->d_queue, 0, sizeof(unsigned) * 2 * dev::kCounterStride));
 #undef DFRG_HIP_B
   // signature for the autotune cache
   {

@@ -198,8 +198,9 @@ int dfrg_se_batch_evals(dfrg_se_batch *b, unsigned long long *evals);
  * tolerance of form 1).  The choice depends on the integral alone, not on the batch. */
 int dfrg_se_batch_variants(dfrg_se_batch *b, int mode, int *variant);
 /* Radial unroll of the mixed path's paired evaluation loop at the current shape: 2 (two radial
- * nodes per step) when the launch puts at most 16 waves on a CU, else 1.  The plain path always
- * uses 1.  Results do not depend on it. */
+ * nodes per step) when the launch puts at most 16 waves on a CU, else 1.  The plain path's general
+ * form always uses 1; its seeded form follows the same rule as the mixed path.  Results do not
+ * depend on it. */
 int dfrg_se_batch_unroll(dfrg_se_batch *b, int *unroll);
 
 /* dfrg_se_batch_run without any allocation.  No counterpart in the reference: it is for callers
