@@ -98,6 +98,19 @@ namespace dfrg
       return y;
     }
 
+    // Sum of one vector by wave_sum8's tree (bitwise its total), in every lane: both cross-row steps
+    // are register swaps instead of wave_sum's LDS permutes.
+    __device__ __forceinline__ double wave_sum1(double v)
+    {
+      double y = pair_sum32(v, v);
+      y = pair_sum16(y, y);
+      y += dpp_f64<0x128>(y); // row_ror:8 pairs lane l with l ^ 8
+      y += dpp_f64<0xB1>(y);  // lane ^ 1
+      y += dpp_f64<0x4E>(y);  // lane ^ 2
+      y += dpp_f64<0x141>(y); // the two quads of each 8 lanes
+      return y;
+    }
+
     // Block sum in a fixed order: wave sums to LDS, then wave 0 adds them in index order.
     // `smem` needs blockDim.x / 64 doubles.  Returns the total to every thread of the block.
     __device__ __forceinline__ double block_sum(double v, double *smem)

@@ -1,0 +1,48 @@
+"""The threshold batch at the sizes where their work split changes, against the oracle.
+
+Tolerance 1e-13: each term differs from the oracle's by a few roundings (the reciprocal within 1 ulp,
+at most five products), and both add positive terms or, near a pole, terms of one sign per node.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-13
+
+
+# register tiles of 64, 128 and 256 nodes and the loop beyond them; groups of eight integrals, one
+# wave, one block of 16 waves, and more groups than resident waves
+@pytest.mark.parametrize("nx", [1, 2, 63, 64, 65, 128, 129, 256, 257, 600])
+@pytest.mark.parametrize("n,k,d", [(1, 1.0, 4), (7, 1e-3, 2), (8, 30.0, 7), (9, 1.0, 3), (1025, 0.2, 5),
+                                   (33003, 1.0, 4)])
+def test_threshold_sizes(gpu, qp, nx, n, k, d):
+    if n > 5000 and nx > 257:
+        n = 5001
+    m2 = np.random.default_rng(n + nx).uniform(-0.9, 4.0, n) * k * k
+    x, w = qp.get_points(nx), qp.get_weights(nx)
+    ref = O.c0_threshold(m2, x, w, 20.0, k, 1.0, d)
+    d_m2, d_x, d_w = (gpu.DeviceArray.from_host(a) for a in (m2, x, w))
+    out = gpu.DeviceArray.from_host(np.full(n + 9, -1.0))
+    for mode in (gpu.FP64, gpu.MIXED):
+        print(f"[case] threshold n={n} nx={nx} k={k} d={d} mode={mode}", flush=True)
+        gpu.threshold_batch(d_m2, d_x, d_w, out, 20.0, k, mode, d)
+        got = out.to_host()
+        assert np.all(got[n:] == -1.0)  # nothing past the last integral
+        assert np.abs(got[:n] / ref - 1).max() <= TOL
+
+
+def test_threshold_special_masses(gpu, qp):
+    # infinite masses give 0, NaN gives NaN; a neighbour in the same group of eight is not touched
+    x, w = qp.get_points(33), qp.get_weights(33)
+    m2 = np.array([0.5, np.inf, np.nan, 1e300, -np.inf, 0.5, 0.25, 0.5, 0.5])
+    d_m2, d_x, d_w = (gpu.DeviceArray.from_host(a) for a in (m2, x, w))
+    out = gpu.DeviceArray(len(m2))
+    print("[case] threshold special masses", flush=True)
+    gpu.threshold_batch(d_m2, d_x, d_w, out, 20.0, 1.0, gpu.FP64, 4)
+    got = out.to_host()
+    ref = O.c0_threshold(np.array([0.5, 0.25]), x, w, 20.0, 1.0, 1.0, 4)
+    assert np.all(got[[1, 3, 4]] == 0.0) and np.isnan(got[2])
+    assert np.abs(got[[0, 5, 7, 8]] / ref[0] - 1).max() <= TOL and abs(got[6] / ref[1] - 1) <= TOL
