@@ -162,7 +162,7 @@ namespace
   }
 
   // ============================================================================================
-  // C2: finite-T two-propagator integrals, one block per integral
+  // finite-T two-propagator integrals, one block per integral
   // ============================================================================================
   struct FTArgs {
     int d, radial_mode, n_int, nx;
@@ -170,28 +170,42 @@ namespace
     const int *m_off, *m_n;
     const double *x, *w;
     double extent, k, pref;
+    double scale, root; // a power of four near 1/k^2, and its root
     double *out;
   };
+
+  // A frequency pair f(q,w) + f(q,-w) = RBdot (d2p + d2m)/(d1^2 d2p d2m) takes one reciprocal of the
+  // product of its denominators (16 VALU against 45 for three IEEE divisions; FP64 mode rcp_f64,
+  // mixed mode the FP32-seeded rcp_seeded).  The denominators are formed times `scale`, so their product
+  // stays in range at any k; scale is a power of two and changes no rounding.
+  template <int MODE> __device__ __forceinline__ double ft_rcp(double d)
+  {
+    return MODE == DFRG_FP64 ? dev::rcp_f64(d) : dev::rcp_seeded(d);
+  }
 
   template <int MODE, int BLOCK> __global__ __launch_bounds__(BLOCK) void ft_kernel(FTArgs A)
   {
     extern __shared__ double sm[];
     const int nx = A.nx;
-    double *s_elw = sm;          // element * weight (plain) or element * weight * RBdot (mixed)
-    double *s_rdot = sm + nx;    // RBdot(q^2)
-    double *s_a1 = sm + 2 * nx;  // q^2 + R(q^2) + m1
-    double *s_a2 = sm + 3 * nx;  // q^2 + |p|^2 + R(q^2 + |p|^2) + m2
-    double *s_red = sm + 4 * nx; // block reduction
+    double *s_f = sm;            // element * weight * RBdot * scale^3
+    double *s_a1 = sm + nx;      // (q^2 + R(q^2) + m1) scale
+    double *s_a2 = sm + 2 * nx;  // (q^2 + |p|^2 + R(q^2 + |p|^2) + m2) scale
+    double *s_red = sm + 3 * nx; // block reduction
     const int i = blockIdx.x;
-    const double k = A.k, k2 = k * k;
-    const double T = A.T[i], p0 = A.p0[i], pa = A.pabs[i], m1 = A.m1[i], m2 = A.m2[i];
+    const double k = A.k, k2 = k * k, sc = A.scale;
+    const double T = A.T[i], pa = A.pabs[i], m1 = A.m1[i], m2 = A.m2[i], p0 = A.p0[i] * A.root;
     const int off = A.m_off[i], nm = A.m_n[i];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    // lanes (as a power of two) a chunk of `rest` Matsubara nodes takes: 64, or for a last chunk of at
+    // most 32 the next power of two, with 64 >> it radial nodes at once, so short rules and remainders
+    // do not leave lanes idle
+    auto log2_lanes = [](int rest) { return rest > 32 ? 6 : 32 - __builtin_clz((rest - 1) | 1); };
     // this lane's first Matsubara node, loaded before the q-only terms so the two loads overlap
     double wn0 = 0.0, wgt0 = 0.0;
-    if (lane < nm) {
-      wn0 = A.mx[off + lane];
-      wgt0 = A.mw[off + lane];
+    const int nl0 = lane & ((1 << log2_lanes(nm)) - 1);
+    if (nl0 < nm) {
+      wn0 = A.mx[off + nl0];
+      wgt0 = A.mw[off + nl0];
     }
     double acc = 0.0;
     // q-only terms, and the zero mode T f(q, 0) of sum = T f(0) + sum_n w_n (f(x_n) + f(-x_n))
@@ -204,66 +218,55 @@ namespace
         q = A.extent * A.x[j];
         el = A.pref * ipow_dev(q, A.d - 2);
       }
-      const double q2 = q * q;
-      const double elw = el * (A.w[j] * A.extent);
-      const double xr = q2 / k2;
-      const double rdot = 2.0 * exp(-xr) * k2 * (1.0 + xr);
-      const double a1 = q2 + k2 * exp(-xr) + m1;
+      const double q2 = q * q, xr = q2 / k2, e = exp(-xr);
+      const double f = el * (A.w[j] * A.extent) * (2.0 * e * k2 * (1.0 + xr)) * sc * sc * sc;
       const double qp2 = q2 + pa * pa;
-      const double a2 = qp2 + k2 * exp(-(qp2 / k2)) + m2;
-      s_elw[j] = MODE == DFRG_FP64 ? elw : elw * rdot;
-      s_rdot[j] = rdot;
+      const double a1 = (q2 + k2 * e + m1) * sc;
+      const double a2 = (qp2 + k2 * exp(-(qp2 / k2)) + m2) * sc;
+      s_f[j] = f;
       s_a1[j] = a1;
       s_a2[j] = a2;
       if (T > 0) {
-        double g10, g20;
-        if (MODE == DFRG_FP64) {
-          g10 = 1.0 / a1;
-          g20 = 1.0 / (p0 * p0 + a2);
-        } else {
-          g10 = dev::rcp_seeded(a1);
-          g20 = dev::rcp_seeded(p0 * p0 + a2);
-        }
-        acc += elw * (T * (rdot * g10 * g10 * g20));
+        const double d2 = p0 * p0 + a2, r = ft_rcp<MODE>(a1 * d2);
+        acc += f * (T * (r * (r * d2)));
       }
     }
     __syncthreads();
-    // Matsubara nodes across the lanes (fixed per lane), radial nodes across the waves; the
-    // q-only terms are wave-uniform LDS reads
+    // Matsubara nodes across the lanes (fixed per lane), radial nodes across the waves; the q terms
+    // are LDS reads shared by the lanes
     constexpr int NW = BLOCK / 64;
     for (int n0 = 0; n0 < nm; n0 += 64) {
-      const int n = n0 + lane;
+      const int rest = nm - n0, lp = log2_lanes(rest);
+      const int n = n0 + (lane & ((1 << lp) - 1));
       if (n >= nm) break;
-      const double wn = n0 == 0 ? wn0 : A.mx[off + n], wgt = n0 == 0 ? wgt0 : A.mw[off + n];
+      const double wn = A.root * (n0 == 0 ? wn0 : A.mx[off + n]), wgt = n0 == 0 ? wgt0 : A.mw[off + n];
       const double dp = wn + p0, dm = -wn + p0;
-      if (MODE == DFRG_FP64) {
-        // the reference's expression tree: three FP64 divisions per pair
-        double s = 0.0;
-#pragma unroll 2
-        for (int j = wv; j < nx; j += NW) {
-          const double a1 = s_a1[j], a2 = s_a2[j], rd = s_rdot[j];
-          const double g1 = 1.0 / (wn * wn + a1), gp = 1.0 / (dp * dp + a2), gm = 1.0 / (dm * dm + a2);
-          s += s_elw[j] * (wgt * (rd * g1 * g1 * gp + rd * g1 * g1 * gm));
-        }
-        acc += s;
-      } else {
-        // f(q,w) + f(q,-w) = RBdot (d2p + d2m) / (d1^2 d2p d2m): one reciprocal per pair, from an
-        // FP32 hardware seed refined in FP64; denominators and products in FP64
-        const double w2 = wn * wn, dp2 = dp * dp, dm2 = dm * dm;
-        double s = 0.0;
+      const double w2 = wn * wn, dp2 = dp * dp, dm2 = dm * dm;
+      double s = 0.0;
+      auto term = [&](int j) {
+        const double a2 = s_a2[j];
+        const double d1 = w2 + s_a1[j];
+        const double d2p = dp2 + a2, d2m = dm2 + a2;
+        const double D2 = d2p * d2m;
+        const double r = ft_rcp<MODE>(d1 * D2);
+        s = fma(s_f[j], (d2p + d2m) * (r * (r * D2)), s);
+      };
+      if (lp == 6) { // one radial node per wave: a uniform loop (28.0 -> 25.8 us below)
 #pragma unroll 4
-        for (int j = wv; j < nx; j += NW) {
-          const double a2 = s_a2[j];
-          const double d1 = w2 + s_a1[j];
-          const double d2p = dp2 + a2, d2m = dm2 + a2;
-          const double D2 = d2p * d2m;
-          const double r = dev::rcp_seeded(d1 * D2);
-          s = fma(s_elw[j], (d2p + d2m) * (r * (r * D2)), s);
-        }
-        acc = fma(wgt, s, acc);
+        for (int j = __builtin_amdgcn_readfirstlane(wv); j < nx; j += NW) term(j);
+      } else {
+        const int G = 64 >> lp;
+#pragma unroll 4
+        for (int j = wv * G + (lane >> lp); j < nx; j += NW * G) term(j);
       }
+      acc = fma(wgt, s, acc);
     }
-    const double tot = dev::block_sum(acc, s_red);
+    double tot = dev::wave_sum1(acc);
+    if (NW > 1) {
+      if (lane == 0) s_red[wv] = tot;
+      __syncthreads();
+      for (int u = 1; wv == 0 && u < NW; ++u) tot += s_red[u];
+    }
     if (threadIdx.x == 0) A.out[i] = tot;
   }
 
@@ -982,8 +985,12 @@ int dfrg_ft_batch(int d, int radial_mode, int n_int, const double *d_T, const do
   DFRG_CHECK_ARG(d_T && d_p0 && d_pabs && d_m1 && d_m2 && d_mx && d_mw && d_m_off && d_m_n && d_x && d_w && d_out,
                  "NULL device pointer");
   FTArgs a{d, radial_mode, n_int, nx, d_T, d_p0, d_pabs, d_m1, d_m2, d_mx, d_mw, d_m_off, d_m_n, d_x, d_w,
-           extent, k, 0.0, d_out};
+           extent, k, 0.0, 1.0, 1.0, d_out};
   a.pref = S_d_host(d - 1) / std::pow(2.0 * kPi, d - 1);
+  if (std::isnormal(k)) {
+    a.root = std::ldexp(1.0, -std::ilogb(k));
+    a.scale = a.root * a.root;
+  }
   // threads per integral: the caller's choice (dfrg_ft_set_block), else enough waves for about
   // two per SIMD over the whole batch, 1 to 8 per integral and not more than radial nodes
   int B = g_ft_block;
@@ -994,7 +1001,7 @@ int dfrg_ft_batch(int d, int radial_mode, int n_int, const double *d_T, const do
     B = 64 * nw;
   }
   hipStream_t s = resolve_stream(stream);
-  const size_t shm = sizeof(double) * (4 * nx + B / 64);
+  const size_t shm = sizeof(double) * (3 * nx + B / 64);
   if (mode == DFRG_FP64) {
     switch (B) {
     case 64: hipLaunchKernelGGL((ft_kernel<DFRG_FP64, 64>), dim3(n_int), dim3(64), shm, s, a); break;

@@ -1,4 +1,4 @@
-"""The threshold batch at the sizes where their work split changes, against the oracle.
+"""The threshold and finite-T batches at the sizes where their work split changes, against the oracle.
 
 Tolerance 1e-13: each term differs from the oracle's by a few roundings (the reciprocal within 1 ulp,
 at most five products), and both add positive terms or, near a pole, terms of one sign per node.
@@ -46,3 +46,39 @@ def test_threshold_special_masses(gpu, qp):
     ref = O.c0_threshold(np.array([0.5, 0.25]), x, w, 20.0, 1.0, 1.0, 4)
     assert np.all(got[[1, 3, 4]] == 0.0) and np.isnan(got[2])
     assert np.abs(got[[0, 5, 7, 8]] / ref[0] - 1).max() <= TOL and abs(got[6] / ref[1] - 1) <= TOL
+
+
+# Matsubara rules around the 64-lane chunk and the powers of two of a last chunk's lane split; nx
+# around the waves' radial strides; scales k far from 1
+@pytest.mark.parametrize("nm", [1, 2, 3, 5, 16, 17, 31, 32, 33, 64, 65, 66, 96, 97, 130])
+@pytest.mark.parametrize("nx,k,radial_mode", [(1, 1.0, 1), (37, 1e-3, 0), (64, 1e18, 1), (65, 1e-20, 0),
+                                              (1024, 1.0, 1)])
+def test_finite_T_sizes(gpu, qp, nm, nx, k, radial_mode):
+    rng = np.random.default_rng(nm + nx)
+    n, d = 9, 4
+    T = k * rng.choice([0.05, 0.1, 0.3], n)
+    T[3] = 0.0  # no zero mode
+    p0 = 2 * np.pi * T * rng.integers(0, 5, n)
+    pabs = 2.0 * k * rng.random(n)
+    m1, m2 = k * k * rng.uniform(-0.5, 3, n), k * k * rng.uniform(-0.5, 3, n)
+    lens = np.array([nm, max(1, nm - 1), nm + 1])
+    off = np.concatenate([[0], np.cumsum(lens)[:-1]])
+    rules = [(2 * np.pi * 0.1 * k * np.arange(1, m + 1), np.full(m, 0.1 * k)) for m in lens]
+    sel = rng.integers(0, 3, n)
+    x, w = qp.get_points(nx), qp.get_weights(nx)
+    extent = 6.0 * k if radial_mode else 20.0
+    ref = O.c2_finiteT(T, p0, pabs, m1, m2, [rules[s] for s in sel], x, w, extent, k, 1.0, d, radial_mode)
+    A = gpu.DeviceArray.from_host
+    dev = {"T": A(T), "p0": A(p0), "pabs": A(pabs), "m1": A(m1), "m2": A(m2),
+           "mx": A(np.concatenate([r[0] for r in rules])), "mw": A(np.concatenate([r[1] for r in rules])),
+           "m_off": A(off[sel].astype(np.int32)), "m_n": A(lens[sel].astype(np.int32)), "x": A(x), "w": A(w)}
+    out = gpu.DeviceArray(n)
+    try:
+        for block in (0, 64, 256):
+            gpu.ft_set_block(block)
+            for mode in (gpu.FP64, gpu.MIXED):
+                print(f"[case] finite-T nm={nm} nx={nx} k={k} block={block} mode={mode}", flush=True)
+                gpu.ft_batch(dev, out, extent, k, mode, d, radial_mode)
+                assert np.abs(out.to_host() / ref - 1).max() <= TOL
+    finally:
+        gpu.ft_set_block(0)
