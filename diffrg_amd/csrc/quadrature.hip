@@ -1,19 +1,21 @@
 // quadrature.hip -- FP64 quadrature rules generated on the GPU, and the provider cache.
 //
-// Gauss-Legendre: one lane per root, Newton iteration on the Legendre three-term recurrence in
-// double-double arithmetic, so that nodes near 0 and 1 keep full relative precision after the
-// map t = (1 -+ z)/2.  Replaces GSL's gsl_integration_fixed_legendre (quadrature.cu:23-58).
+// Gauss-Legendre: one lane per root.  FP64 Newton iterations on the Legendre three-term recurrence
+// bring the root to a few roundings; one compensated pass of the same recurrence (its rounding
+// errors carried exactly and propagated alongside) then gives P_n there to twice FP64's digits, so
+// that nodes near 0 and 1 keep full relative precision after the map t = (1 -+ z)/2.  Replaces GSL's
+// gsl_integration_fixed_legendre (quadrature.cu:23-58).
 //
 // Matsubara (Monien, Math. Comp. 79, 857 (2010); matsubara.cu:33-85): the Jacobi matrix of the
-// recurrence a_j, b_j is built on the device; lane i finds the i-th smallest eigenvalue by Sturm
-// bisection and the first component of its eigenvector from a twisted factorisation
+// recurrence a_j, b_j; wave i finds the i-th smallest eigenvalue by multisection on the Sturm count
+// (64 points per round) and the first component of its eigenvector from a twisted factorisation
 // (Parlett & Dhillon's twisted LDL^T / UDU^T, the core of MRRR).  The reference diagonalises the
 // same matrix with the sequential implicit-QL routine IMTQLX (diagonalization.hh:34-145); the
 // parallel form is at least as accurate on this graded matrix.
 #include "internal.hh"
 #include "dfrg/device.hh"
 
-// The double-double arithmetic below relies on error-free transformations; fusing a product
+// The compensated recurrence below relies on error-free transformations; fusing a product
 // into a later sum (FP contraction, on by default for device code) would break them.
 #pragma clang fp contract(off)
 
@@ -25,191 +27,260 @@ namespace dfrg
 {
   namespace
   {
-    // ---------------------------------------------------------------------------------------
-    // double-double arithmetic (Dekker / Knuth error-free transformations)
-    // ---------------------------------------------------------------------------------------
-    struct dd {
-      double hi, lo;
-    };
-    __device__ __forceinline__ dd quick_two_sum(double a, double b)
-    {
-      const double s = a + b;
-      return {s, b - (s - a)};
-    }
-    __device__ __forceinline__ dd two_sum(double a, double b)
+    // a + b = sum + err exactly (Knuth)
+    __device__ __forceinline__ double two_sum(double a, double b, double &err)
     {
       const double s = a + b;
       const double bb = s - a;
-      return {s, (a - (s - bb)) + (b - bb)};
+      err = (a - (s - bb)) + (b - bb);
+      return s;
     }
-    __device__ __forceinline__ dd dd_add(dd a, dd b)
-    {
-      dd s = two_sum(a.hi, b.hi);
-      const dd t = two_sum(a.lo, b.lo);
-      s.lo += t.hi;
-      s = quick_two_sum(s.hi, s.lo);
-      s.lo += t.lo;
-      return quick_two_sum(s.hi, s.lo);
-    }
-    __device__ __forceinline__ dd dd_neg(dd a) { return {-a.hi, -a.lo}; }
-    __device__ __forceinline__ dd dd_sub(dd a, dd b) { return dd_add(a, dd_neg(b)); }
-    __device__ __forceinline__ dd dd_mul(dd a, dd b)
-    {
-      const double p = a.hi * b.hi;
-      double e = fma(a.hi, b.hi, -p);
-      e += a.hi * b.lo + a.lo * b.hi;
-      return quick_two_sum(p, e);
-    }
-    __device__ __forceinline__ dd dd_mul_d(dd a, double b)
-    {
-      const double p = a.hi * b;
-      double e = fma(a.hi, b, -p);
-      e += a.lo * b;
-      return quick_two_sum(p, e);
-    }
-    __device__ __forceinline__ dd dd_div(dd a, dd b)
-    {
-      const double q1 = a.hi / b.hi;
-      dd r = dd_sub(a, dd_mul_d(b, q1));
-      const double q2 = r.hi / b.hi;
-      r = dd_sub(r, dd_mul_d(b, q2));
-      const double q3 = r.hi / b.hi;
-      return dd_add(quick_two_sum(q1, q2), dd{q3, 0.0});
-    }
-    __device__ __forceinline__ dd dd_from(double a) { return {a, 0.0}; }
 
-    // P_n(z) and P_n'(z) by the three-term recurrence, in double-double.
-    __device__ void legendre_dd(int n, dd z, dd *pn, dd *dpn)
+    // Rules of a few dozen to a few hundred nodes run on a handful of waves, so the serial recurrence
+    // over the order bounds the kernel: what counts is its dependent chain per degree.  With 1/j
+    // tabulated in LDS, an FP64 step is one dependent FMA, and the compensated step has four
+    // dependent operations with its error terms beside them; the earlier form took every Newton step
+    // in double-double with a three-division quotient per degree.  Order 128: 293 -> 16.8 us, 32: 86 ->
+    // 6.6, 1024: 1972 -> 96.5.
+    constexpr int kGlBlock = 64;
+    __global__ __launch_bounds__(kGlBlock) void gl_kernel(int n, double *x, double *w)
     {
-      dd p0 = dd_from(1.0), p1 = z;
+      extern __shared__ double2 s_inv[]; // 1/j = x + y at j - 1, j <= n
+      for (int j = 1 + threadIdx.x; j <= n; j += kGlBlock) {
+        const double hi = 1.0 / j;
+        s_inv[j - 1] = make_double2(hi, fma(-hi, (double)j, 1.0) * hi);
+      }
+      __syncthreads();
+      const int i = blockIdx.x * kGlBlock + threadIdx.x;
+      const bool own = i < (n + 1) / 2;
+      // i-th root from the top; Tricomi's initial guess.  Odd n: the middle root is 0 exactly.
+      const double dn = n;
+      const bool middle = (n & 1) && i == n / 2;
+      double z = middle || !own ? 0.0
+                                : (1.0 - (dn - 1.0) / (8.0 * dn * dn * dn)) * cos(dev::pi * (i + 0.75) / (n + 0.5));
+      // Newton in FP64: P_j = (2 - 1/j) z P_{j-1} - (1 - 1/j) P_{j-2};  P_n' = n (z P_n - P_{n-1})/(z^2 - 1)
+      for (int it = 0; it < 8; ++it) {
+        double p0 = 1.0, p1 = z;
+#pragma unroll 8
+        for (int j = 2; j <= n; ++j) {
+          const double inv = s_inv[j - 1].x;
+          const double p2 = fma((2.0 - inv) * z, p1, -((1.0 - inv) * p0));
+          p0 = p1;
+          p1 = p2;
+        }
+        const double dz = p1 * fma(z, z, -1.0) / (dn * fma(z, p1, -p0));
+        if (n > 1 && own && !middle) z -= dz;
+        // the step leaves about dz^2 n^2/6 near the ends, less elsewhere: below an FP64 rounding
+        if (__builtin_amdgcn_ballot_w64(own && !middle && fabs(dz) * dn > 3e-8) == 0) break;
+      }
+      // one pass at the FP64 root with its rounding errors: with u = z P_{j-1} and t = u - P_{j-2},
+      // P_j = u + t - t/j; e carries the error of P_j through the same recurrence
+      double p0 = 1.0, p1 = z, e0 = 0.0, e1 = 0.0;
+#pragma unroll 4
       for (int j = 2; j <= n; ++j) {
-        const dd t = dd_sub(dd_mul(dd_mul_d(z, 2.0 * j - 1.0), p1), dd_mul_d(p0, j - 1.0));
-        const dd p2 = dd_div(t, dd_from((double)j));
+        const double2 inv = s_inv[j - 1];
+        double dt, ds, dp;
+        const double u = z * p1, du = fma(z, p1, -u);
+        const double t = two_sum(u, -p0, dt);
+        const double v = t * inv.x, dv = fma(t, inv.x, -v);
+        const double s = two_sum(u, t, ds);
+        const double p2 = two_sum(s, -v, dp);
+        const double eu = fma(z, e1, du), et = (eu - e0) + dt;
+        const double ev = fma(et, inv.x, fma(t, inv.y, dv));
+        const double e2 = ((eu + et) - ev) + (ds + dp);
         p0 = p1;
         p1 = p2;
+        e0 = e1;
+        e1 = e2;
       }
-      *pn = p1;
-      // n (z P_n - P_{n-1}) / (z^2 - 1)
-      *dpn = dd_div(dd_mul_d(dd_sub(dd_mul(z, p1), p0), (double)n), dd_sub(dd_mul(z, z), dd_from(1.0)));
-    }
-
-    __global__ void gl_kernel(int n, double *x, double *w)
-    {
-      const int i = blockIdx.x * blockDim.x + threadIdx.x;
-      if (i >= (n + 1) / 2) return;
-      // i-th root from the top; Tricomi-type initial guess
-      dd z = dd_from(cos(dev::pi * (i + 0.75) / (n + 0.5)));
-      dd pn, dpn;
-      for (int it = 0; it < 12; ++it) {
-        legendre_dd(n, z, &pn, &dpn);
-        const dd dz = dd_div(pn, dpn);
-        z = dd_sub(z, dz);
-        if (fabs(dz.hi) <= 1e-31 * fmax(fabs(z.hi), 1e-3)) break;
+      if (!own) return;
+      const double f = n > 1 ? p1 + e1 : 0.0;
+      if (n == 1) {
+        p0 = 1.0;
+        e0 = 0.0;
       }
-      legendre_dd(n, z, &pn, &dpn);
-      const dd one = dd_from(1.0);
-      // weight on [0,1]: 1 / ((1 - z^2) P_n'(z)^2)
-      const dd wz = dd_div(one, dd_mul(dd_sub(one, dd_mul(z, z)), dd_mul(dpn, dpn)));
-      const dd xhi = dd_mul_d(dd_add(one, z), 0.5);
-      const dd xlo = dd_mul_d(dd_sub(one, z), 0.5);
-      x[n - 1 - i] = xhi.hi;
-      x[i] = xlo.hi;
-      w[n - 1 - i] = wz.hi;
-      w[i] = wz.hi;
-      if ((n & 1) && i == n / 2) x[i] = 0.5;
+      // 1 - z and 1 + z exactly, and the root's correction d: Newton with its second-order term
+      // (P'' = 2 z P'/(1 - z^2) at a root)
+      double om_e, op_e;
+      const double om = two_sum(1.0, -z, om_e), op = two_sum(1.0, z, op_e);
+      const double q = om * op;                                // 1 - z^2
+      const double pm = p0 + e0;
+      const double d1 = -f * q / (dn * fma(-z, f, pm)); // -P/P'
+      const double d = middle ? 0.0 : d1 - d1 * d1 * (z / q);
+      const double om_l = om_e - d, op_l = op_e + d;
+      const double xlo = om + om_l, xhi = op + op_l; // 1 - z*, 1 + z*
+      // weight on [0,1]: 1 / ((1 - z^2) P_n'(z)^2) = (1 - z^2) / (n P_{n-1})^2 at the root z* = z + d, in
+      // twice FP64's digits up to the last division: P_{n-1} moved by its Taylor series (P'/P =
+      // n (z - P_n/P)/(1 - z^2) =: g, P''/P = (2 z g - n (n - 1))/(1 - z^2))
+      const double g = dn * (z - f / pm) / q, h = 0.5 * (2.0 * z * g - dn * (dn - 1.0)) / q;
+      const double pm_l = fma(pm, fma(h, d, g) * d, e0);
+      const double t = dn * p0, t_l = fma(dn, pm_l, fma(dn, p0, -t));
+      const double den = t * t, den_l = fma(t, t, -den) + (2.0 * t * t_l + t_l * t_l);
+      const double num = q, num_l = fma(om, op, -q) + (om * op_l + om_l * op);
+      const double w0 = num / den;
+      const double wz = w0 + (fma(-w0, den, num) + fma(-w0, den_l, num_l)) / (den + den_l);
+      x[n - 1 - i] = 0.5 * xhi;
+      x[i] = middle ? 0.5 : 0.5 * xlo;
+      w[n - 1 - i] = wz;
+      w[i] = wz;
     }
 
     // ---------------------------------------------------------------------------------------
     // Monien rule
     // ---------------------------------------------------------------------------------------
-    __device__ __forceinline__ int sturm_count_below(const double *a, const double *e2, int n, double x)
+    // Number of eigenvalues of the tridiagonal (a, e^2) below x: negative pivots of its LDL^T
+    // factorisation.
+    __device__ __forceinline__ int sturm_count_below(const double2 *m, int n, double x)
     {
-      int c = 0;
-      double q = a[0] - x;
-      c += q < 0.0;
-      for (int i = 1; i < n; ++i) {
+      double q = m[0].x - x;
+      int c = q < 0.0;
+#pragma unroll 4
+      for (int j = 1; j < n; ++j) {
         if (q == 0.0) q = 1e-300;
-        q = (a[i] - x) - e2[i - 1] / q;
+        q = (m[j].x - x) - m[j].y / q;
         c += q < 0.0;
       }
       return c;
     }
 
-    // One block; n <= 1024 lanes; scratch holds 2 n^2 doubles (per-lane twisted factorisation).
-    __global__ void matsubara_kernel(int n, double T, double *x_out, double *w_out, double *scratch)
+    // The same count by the sign changes of the Sturm sequence p_j = (a_j - x) p_{j-1} - e_{j-1}^2 p_{j-2},
+    // whose ratios are those pivots: one dependent FMA per step instead of a division, and the two agree
+    // but for x within about 1e-12 of an eigenvalue.  The pair is rescaled by a power of two every
+    // eight steps; the entries (e^2 down to 1e-13 at n = 1024) cannot take it out of range in between.
+    __device__ __forceinline__ int sturm_count_quick(const double2 *m, int n, double x)
+    {
+      double p0 = 1.0, p1 = m[0].x - x;
+      int c = p1 < 0.0;
+      auto step = [&](int j) {
+        const double2 ae = m[j]; // a_j, e_{j-1}^2
+        double p2 = fma(ae.x - x, p1, -(ae.y * p0));
+        if (p2 == 0.0) p2 = copysign(1e-200, p1); // a zero pivot counts as positive, the next as negative
+        c += (unsigned)(__double2hiint(p2) ^ __double2hiint(p1)) >> 31;
+        p0 = p1;
+        p1 = p2;
+      };
+      int j = 1;
+      for (; j + 8 <= n; j += 8) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) step(j + u);
+        const int ex = -max(__builtin_amdgcn_frexp_exp(p0), __builtin_amdgcn_frexp_exp(p1));
+        p0 = ldexp(p0, ex);
+        p1 = ldexp(p1, ex);
+      }
+      for (; j < n; ++j) step(j);
+      return c;
+    }
+
+    // One wave per node: every block forms the matrix in its LDS.  Rounds of 64 points shrink the bracket
+    // about 64-fold each, nine quick counts and two with pivots against 70 bisection steps with pivots,
+    // whose division chain bounded the kernel (all nodes had shared one block); the two halves of the
+    // twisted factorisation run on two lanes.  A call for 66 nodes, launch to synchronised
+    // result, 414 -> 87 us, for 32 nodes 213 -> 75, most of what is left on the host.
+    __global__ __launch_bounds__(64) void matsubara_kernel(int n, double T, double *x_out, double *w_out)
     {
       extern __shared__ double sm[];
-      double *a = sm;          // diagonal
-      double *e = sm + n;      // off-diagonal, e[j] couples j and j+1
-      double *e2 = sm + 2 * n; // e^2
+      double2 *m = (double2 *)sm; // a_j, e_{j-1}^2
+      double *e = sm + 2 * n;     // off-diagonal, e[j] couples j and j+1
+      double *d = sm + 3 * n, *dp = sm + 4 * n;
       const double pi = dev::pi;
-      for (int j = threadIdx.x; j < n; j += blockDim.x) {
+      const int lane = threadIdx.x, k = blockIdx.x;
+      for (int j = lane; j < n; j += 64) {
         const double j1 = j + 1;
         double aj = 2.0 * (pi * pi) / (4 * j + 1) / (4 * j + 5);
         if (j == 0) aj = (pi * pi) / 15.0;
-        a[j] = aj;
         const double bj = (pi * (pi * (pi * pi))) / ((4 * j1 - 1) * (4 * j1 + 3)) / ((4 * j1 + 1) * (4 * j1 + 1));
         const double ej = (j < n - 1) ? sqrt(bj) : 0.0;
         e[j] = ej;
+        m[j].x = aj;
+        if (j + 1 < n) m[j + 1].y = ej * ej;
+        if (j == 0) m[0].y = 0.0;
       }
       __syncthreads();
-      for (int j = threadIdx.x; j < n; j += blockDim.x) e2[j] = e[j] * e[j];
-      __syncthreads();
-
-      const int k = threadIdx.x;
-      if (k >= n) return;
-      // Gershgorin interval
-      double lo = 1e300, hi = -1e300;
-      for (int j = 0; j < n; ++j) {
-        const double r = (j > 0 ? fabs(e[j - 1]) : 0.0) + (j < n - 1 ? fabs(e[j]) : 0.0);
-        lo = fmin(lo, a[j] - r);
-        hi = fmax(hi, a[j] + r);
+      // k-th smallest eigenvalue, 64 points per round: count(x) > k  <=>  lambda_k < x.  All lie in (0, 2)
+      // (Gershgorin); the first round's points are geometric, as the eigenvalues fall like 1/i^2 down to
+      // n^-4.
+      double lo = 0.0, hi = 2.0;
+      auto narrow = [&](double x, int count) {
+        const unsigned long long above = __builtin_amdgcn_ballot_w64(count > k);
+        const int f = above ? __builtin_ctzll(above) : 64; // first point above the eigenvalue
+        if (f < 64) hi = dev::lane_value(x, f);
+        if (f > 0) lo = dev::lane_value(x, f - 1);
+        return f;
+      };
+      {
+        const double x = exp2(-40.0 + (lane + 1) * (41.0 / 65.0));
+        narrow(x, sturm_count_quick(m, n, x));
       }
-      // k-th smallest eigenvalue: count(x) > k  <=>  lambda_k < x
-      for (int it = 0; it < 256; ++it) {
+      for (int it = 0; it < 16 && hi - lo > 0x1p-40 * hi; ++it) {
+        const double x = fma(hi - lo, (lane + 1) * (1.0 / 65.0), lo);
+        narrow(x, sturm_count_quick(m, n, x));
+      }
+      // the last digits by the pivots, as the reference's accuracy is theirs: from a bracket of 1e-12 about
+      // the quick count's value, moved outwards while the pivots' eigenvalue is not in it
+      double w = 0x1p-41 * hi;
+      lo -= w;
+      hi += w;
+      for (int it = 0; it < 16; ++it) {
         const double mid = 0.5 * (lo + hi);
-        if (mid <= lo || mid >= hi) break;
-        if (sturm_count_below(a, e2, n, mid) > k)
-          hi = mid;
-        else
-          lo = mid;
+        if (mid <= lo || mid >= hi || hi - lo <= 0x1p-51 * hi) break;
+        const double x = fma(hi - lo, lane * (1.0 / 63.0), lo); // both ends among the points
+        const double l0 = lo, h0 = hi;
+        const int f = narrow(x, sturm_count_below(m, n, x));
+        w *= 16.0;
+        if (f == 0) lo = l0 - w;  // hi became the old lower end
+        if (f == 64) hi = h0 + w; // lo became the old upper end
       }
       const double lam = 0.5 * (lo + hi);
 
-      // twisted factorisation at lam: top-down pivots d, bottom-up pivots dp
-      double *d = scratch + (size_t)k * 2 * n;
-      double *dp = d + n;
-      d[0] = a[0] - lam;
-      for (int j = 1; j < n; ++j) {
-        const double prev = d[j - 1] != 0.0 ? d[j - 1] : 1e-300;
-        d[j] = (a[j] - lam) - e2[j - 1] / prev;
+      // twisted factorisation at lam: top-down pivots d on lane 0, bottom-up pivots dp on lane 1
+      {
+        double *out = lane == 0 ? d : dp;
+        double q = m[lane == 0 ? 0 : n - 1].x - lam;
+        if (lane < 2) out[lane == 0 ? 0 : n - 1] = q;
+#pragma unroll 4
+        for (int j = 1; j < n; ++j) {
+          const int i = lane == 0 ? j : n - 1 - j;
+          q = fma(-m[lane == 0 ? i : i + 1].y, dev::rcp_f64(q != 0.0 ? q : 1e-300), m[i].x - lam);
+          if (lane < 2) out[i] = q;
+        }
       }
-      dp[n - 1] = a[n - 1] - lam;
-      for (int j = n - 2; j >= 0; --j) {
-        const double next = dp[j + 1] != 0.0 ? dp[j + 1] : 1e-300;
-        dp[j] = (a[j] - lam) - e2[j] / next;
-      }
-      int r = 0;
-      double gmin = 1e300;
-      for (int j = 0; j < n; ++j) {
-        const double g = fabs(d[j] + dp[j] - (a[j] - lam));
+      __syncthreads();
+      // twist index: the smallest gamma_j, the first of equal ones
+      int r = n;
+      double gmin = INFINITY;
+      for (int j = lane; j < n; j += 64) {
+        const double g = fabs(d[j] + dp[j] - (m[j].x - lam));
         if (g < gmin) {
           gmin = g;
           r = j;
         }
       }
-      // eigenvector with z_r = 1; components outward from the twist index
-      double z = 1.0, s = 1.0, z0 = (r == 0) ? 1.0 : 0.0;
-      for (int j = r - 1; j >= 0; --j) {
-        z = -(e[j] / (d[j] != 0.0 ? d[j] : 1e-300)) * z;
-        s += z * z;
-        if (j == 0) z0 = z;
+      for (int o = 32; o; o >>= 1) {
+        const double g = __shfl_xor(gmin, o);
+        const int ro = __shfl_xor(r, o);
+        if (g < gmin || (g == gmin && ro < r)) {
+          gmin = g;
+          r = ro;
+        }
       }
-      z = 1.0;
-      for (int j = r + 1; j < n; ++j) {
-        z = -(e[j - 1] / (dp[j] != 0.0 ? dp[j] : 1e-300)) * z;
-        s += z * z;
+      r = __builtin_amdgcn_readfirstlane(r < n ? r : 0);
+      // eigenvector with z_r = 1: ratios of neighbouring components (into d), then their products outward
+      // from the twist index, downward indices on lane 0, upward ones on lane 1
+      for (int j = lane; j < n; j += 64) {
+        const double p = j < r ? d[j] : dp[j];
+        d[j] = -((j < r ? e[j] : j > 0 ? e[j - 1] : 0.0) / (p != 0.0 ? p : 1e-300));
       }
+      __syncthreads();
+      double z = 1.0, s = 0.0;
+      const int steps = lane == 0 ? r : n - 1 - r;
+#pragma unroll 4
+      for (int j = 1; j <= steps; ++j) {
+        z *= d[lane == 0 ? r - j : r + j];
+        s = fma(z, z, s);
+      }
+      const double z0 = dev::lane_value(z, 0);
+      s = 1.0 + dev::lane_value(s, 0) + dev::lane_value(s, 1);
+      if (lane != 0) return;
       const double mu0 = (pi * pi) / 6.0;
       const double wk = mu0 * (z0 * z0 / s);
       // normalise the weights and scale the nodes (matsubara.cu:78-84)
@@ -240,6 +311,9 @@ namespace dfrg
       if (i < n) b[i] = (float)a[i];
     }
 
+    // LDS of gl_kernel: the reciprocals of 1..order (64 KB at 4096, the largest order)
+    size_t gl_shared(int order) { return sizeof(double2) * order; }
+
     bool is_close_abs(double a, double b, double eps)
     {
       const double diff = std::fabs(a - b);
@@ -269,9 +343,8 @@ int dfrg_gl_generate(int order, double *d_x, double *d_w, void *stream)
   DFRG_CHECK_ARG(order >= 1 && order <= 4096, "Gauss-Legendre order %d out of range [1,4096]", order);
   DFRG_CHECK_ARG(d_x && d_w, "output pointers are NULL");
   const int roots = (order + 1) / 2;
-  const int block = 64;
-  hipLaunchKernelGGL(gl_kernel, dim3((roots + block - 1) / block), dim3(block), 0, resolve_stream(stream), order,
-                     d_x, d_w);
+  hipLaunchKernelGGL(gl_kernel, dim3((roots + kGlBlock - 1) / kGlBlock), dim3(kGlBlock), gl_shared(order),
+                     resolve_stream(stream), order, d_x, d_w);
   DFRG_LAUNCHED("gl_kernel");
   return DFRG_OK;
 }
@@ -296,7 +369,7 @@ int dfrg_matsubara_generate(double T, double E, int step, int min_size, int max_
     const int h = m / 2;
     double *g = nullptr;
     DFRG_HIP(hipMallocAsync((void **)&g, sizeof(double) * 2 * h, s));
-    hipLaunchKernelGGL(gl_kernel, dim3((h + 1) / 2 / 64 + 1), dim3(64), 0, s, h, g, g + h);
+    hipLaunchKernelGGL(gl_kernel, dim3((h + 1) / 2 / kGlBlock + 1), dim3(kGlBlock), gl_shared(h), s, h, g, g + h);
     DFRG_LAUNCHED("gl_kernel");
     hipLaunchKernelGGL(matsubara_vacuum_kernel, dim3(h / 64 + 1), dim3(64), 0, s, h, E, g, g + h, d_x, d_w);
     DFRG_LAUNCHED("matsubara_vacuum_kernel");
@@ -309,12 +382,8 @@ int dfrg_matsubara_generate(double T, double E, int step, int min_size, int max_
   m = std::max(min_size, std::min(max_size, m));
   DFRG_CHECK_ARG(m >= 1 && m <= 1024, "Matsubara rule size %d out of range [1,1024]", m);
   DFRG_CHECK_ARG(m <= cap, "Matsubara rule of %d nodes exceeds capacity %d", m, cap);
-  double *scratch = nullptr;
-  DFRG_HIP(hipMallocAsync((void **)&scratch, sizeof(double) * 2 * (size_t)m * m, s));
-  const int block = ((m + 63) / 64) * 64;
-  hipLaunchKernelGGL(matsubara_kernel, dim3(1), dim3(block), 3 * m * sizeof(double), s, m, T, d_x, d_w, scratch);
+  hipLaunchKernelGGL(matsubara_kernel, dim3(m), dim3(64), 5 * m * sizeof(double), s, m, T, d_x, d_w);
   DFRG_LAUNCHED("matsubara_kernel");
-  DFRG_HIP(hipFreeAsync(scratch, s));
   DFRG_HIP(hipStreamSynchronize(s));
   *size = m;
   if (T_rule) *T_rule = T;
