@@ -10,16 +10,14 @@
 // point and RK stage.  u', u'' are second-order finite differences (one-sided at the ends).
 //
 // Device layout: every resident flow owns 2 n doubles in one HBM pool (u after even and after odd
-// steps) and a slot in SoA descriptor arrays.  The host cuts the resident flows into runs of
-// consecutive grid points; one launch advances every run by a whole RK4 step, one workgroup per
-// run, evaluating the stages outside the run as far as the next stages' stencils reach
-// (flow_step_kernel), each wave two grid points at a time (one Gauss-Legendre node per lane, the
-// four node sums reduced together across lanes).  steps_per_launch steps are captured into one hipGraph.  A flow's step
-// index is the launch's base step plus the step within the graph minus the base step at its
-// admission, so flows admitted at different times share the graph and a finished flow simply
-// stops updating.  The graph's last node advances the device copy
-// of the base step, which the host mirrors.  Between graph launches the host retires
-// finished and non-finite flows and admits queued ones while their HBM footprint fits the budget.
+// steps).  The host cuts the resident flows into runs of consecutive grid points; one launch
+// advances every run by a whole RK4 step, one workgroup per run, evaluating the stages outside the
+// run as far as the next stages' stencils reach (flow_step_kernel).  steps_per_launch steps are
+// captured into one hipGraph.  A flow's step index is the launch's base step plus the step within
+// the graph minus the base step at its admission, so flows admitted at different times share the
+// graph and a finished flow simply stops updating.  The graph's last node advances the device copy
+// of the base step, which the host mirrors.  Between graph launches the host retires finished and
+// non-finite flows and admits queued ones while their HBM footprint fits the budget.
 //
 // Node factors: with x_j the GL nodes, xr_j = x_j x_extent, the regulator terms are
 // q^2 = k^2 xr, R = k^2 e^-xr, RBdot = 2 k^2 e^-xr (1 + xr) and the d = 3 element times weight is
@@ -42,54 +40,196 @@ using namespace dfrg;
 
 namespace
 {
-  constexpr int kFlowGrid = 1024; // workgroups per step launch, grid-stride over runs
   constexpr double kPi = 3.14159265358979323846;
+  constexpr double kLog2e = 1.4426950408889634074;
 
   // A run of consecutive grid points [a, b) of one resident flow, which one workgroup advances by
-  // a whole RK4 step.  Runs are at least 2 points long (the one-sided stencils at the grid ends
-  // then find their points in the previous stage's range) and at most kMaxRun.
+  // a whole RK4 step, with the flow's parameters (one record per run, so a step's loads depend on
+  // it alone).  Runs are at least 2 points long (the one-sided stencils at the grid ends then find
+  // their points in the previous stage's range).
   struct FlowRun {
     int slot, a, b, n, off, admit;
+    double h, i2h, ih2; // grid spacing, 1/(2 h), 1/h^2
+    double T, N;        // temperature, O(N)
+    double m2_0, lam;   // initial condition u(rho) = m2_0 + lam/2 rho (step 0 starts from it)
   };
 
-  constexpr int kRunBlock = 512;                  // threads per workgroup: 8 waves share a run
+  constexpr int kRunBlock = 1024;                 // threads per workgroup: 16 waves share a run
   constexpr int kHalo = 3;                        // stages 1-3 are also evaluated this far outside the run
-  constexpr int kMaxRun = 256;                    // longest run
+  constexpr int kMaxRun = 250;                    // longest run
   constexpr int kSpan = kMaxRun + 2 * (kHalo + 1); // the run and the stencil reach of its stage 1
-  // grid points a wave evaluates together: 2 (rather than 4) balances a stage's points over the 8
-  // waves at short runs; each node sum gets the same add tree either way (dev::wave_sum4)
-  constexpr int kGroup = 2;
+  // run lengths whose first stage (6 points more) fills whole waves on the four SIMDs
+  constexpr int kRunLengths[] = {2, 6, 10, 18, 26, 42, 58, 74, 90, 106, 122, 154, 186, 218, 250};
+  constexpr int kMaxFlowGrid = 1024;              // most workgroups of a step launch, grid-stride over runs
+  constexpr int kFlowGraphs = 5;                  // step graphs, with grids of 64, 128, ... kMaxFlowGrid
+  static_assert(64 << (kFlowGraphs - 1) == kMaxFlowGrid);
 
   struct FlowDev {
-    int *status, *bad;    // per slot; status 0 idle, 1 running (host-owned)
-    double *h, *T, *N;    // per slot: grid spacing, temperature, O(N)
-    double *m2_0, *lam;   // per slot: initial condition u(rho) = m2_0 + lam/2 rho (step 0 reads it)
+    int *bad;             // per slot: a non-finite value appeared
     FlowRun *runs;        // every resident flow cut into runs
     int *n_runs;          // device copy of the run count
     int *base;            // global step index of the first step of this launch
     double *pool;         // state: u at even steps | u at odd steps, per flow
-    const double *A, *D;  // node factors (header comment)
+    const double2 *nodes; // node factors (A_j, D_j/4) (header comment), padded to a multiple of 64 with
+                          // (1e30, 0), whose terms are zeros
+    const double *exp2t;  // 2^(j/512), j = 0..511
     const double *kt;     // k at (step, stage point): 3 per step, t, t + dt/2, t + dt
     int nx, n_steps;
     double dt;
   };
-  // S2(E) = coth(E/2T)/(4E^3) + csch^2(E/2T)/(8 T E^2) with e = exp(-E/T), coth = (1+e)/(1-e),
-  // csch^2 = 4e/(1-e)^2, put over one denominator:
-  //   S2 = (2 T (1+e)(1-e) + 4 e E) / (8 T E^3 (1-e)^2),   E = sqrt(E2).
-  // FP64-accurate seeded forms instead of library calls: y = 1/E from an FP32 rsqrt seed and one
-  // Newton step, E = E2 y; e from the 1/64-grid table and a degree-6 polynomial; the denominator as
-  // the product of 1/(8T), y^3 and the seeded reciprocal of (1-e), squared, so no factor leaves the
-  // FP32 range of the seeds.  1 - e loses relative accuracy only as E/T -> 0 (absolute error
-  // ~1e-16 against 1 - e ~ E/T).  Relative error of S2 ~1e-14.
-  __device__ __forceinline__ double bose_S2(double E2, double T, double inv_8T, double inv_T,
-                                            const double *exp2t)
+  // 2^(a b/512) for |a b| < 2^30: exp2t[j] = 2^(j/512), dev::exp2_tab's rounding, and 2^(f/512) - 1 =
+  // f P(f) with P of degree 3 (remainder 1.3e-19).
+  constexpr int kFlowExp = 512;
+  __device__ __forceinline__ double exp2_tab512(double a, double b, const double *exp2t)
+  {
+    constexpr double kRound = 6755399441055744.0;
+    const double sh = fma(a, b, kRound);
+    const int jn = __double2loint(sh);
+    const double f = fma(a, b, -(sh - kRound));
+    double p = fma(f, 1.399622015673666e-13, 4.1353784454173436e-10);
+    p = fma(p, f, 9.163913992275265e-07);
+    p = fma(p, f, 0.001353803087031143);
+    const double c = exp2t[jn & (kFlowExp - 1)];
+    return ldexp(fma(c * f, p, c), jn >> 9);
+  }
+
+  // The temperature's factors in bose_4S2.
+  struct Bose {
+    double two_inv_T, exp_scale, E_max; // 2/T, -512 log2(e)/T, 1000 T
+    __device__ __forceinline__ explicit Bose(double T)
+    {
+      const double inv_T = 1.0 / T;
+      two_inv_T = 2.0 * inv_T;
+      exp_scale = -512.0 * kLog2e * inv_T;
+      E_max = 1000.0 * T;
+    }
+  };
+  // 4 S2(E) with S2 = coth(E/2T)/(4E^3) + csch^2(E/2T)/(8 T E^2), e = exp(-E/T), coth = (1+e)/(1-e),
+  // csch^2 = 4e/(1-e)^2, r = 1/(1-e) and y = 1/E:
+  //   4 S2 = y^3 r^2 (1 - e^2 + 2 (E/T) e),
+  // by FP64 forms instead of library calls: y and r from FP32 hardware seeds and one Newton step, e by
+  // table (E/T beyond 1000 gives 0 through the exponent).  1 - e loses relative accuracy only as
+  // E/T -> 0 (absolute error ~1e-16 against 1 - e ~ E/T).  Relative error ~1e-14.  E2 <= 0 gives NaN.
+  // 38 VALU instructions against 47 with the temperature's factors inside and a 64-entry table.  (FP64
+  // seeds would take 32, but a flow can carry the 1e-14 they differ by to 3e-11 in its final u.)
+  __device__ __forceinline__ double bose_4S2(double E2, const Bose &B, const double *exp2t)
   {
     const double y = dev::rsqrt_seeded(E2);
-    const double E = E2 * y;
-    const double e = dev::exp_neg_tab(E * inv_T, exp2t), ome = 1.0 - e;
-    const double num = fma(2.0 * T * (1.0 + e), ome, 4.0 * e * E);
-    const double r = dev::rcp_seeded(ome);
-    return num * inv_8T * (y * y * y) * (r * r);
+    const double E = fmin(E2 * y, B.E_max);
+    const double e = exp2_tab512(E, B.exp_scale, exp2t);
+    const double r = dev::rcp_seeded(1.0 - e);
+    const double q = fma(B.two_inv_T, E * e, fma(-e, e, 1.0));
+    return (y * y * y) * (r * r) * q;
+  }
+
+  // a + b with no product fused into it
+  __device__ __forceinline__ double add_plain(double a, double b)
+  {
+#pragma clang fp contract(off)
+    return a + b;
+  }
+
+  // The lanes of one grid point: NL lanes for the threshold integral at u (kind 0), the next NL for
+  // the one at u + 2 rho u' (kind 1); a lane sums 64/NL nodes of each chunk of 64.
+  // Node sums are one tree over the bits of the node index, 5, 4, 3 (in the lane or across lanes,
+  // by NL), then 0, 1, 2 across eight lanes, so a sum's bits do not depend on NL.
+  template <int NL> __device__ __forceinline__ double node_tree(double (&t)[NL == 32 ? 2 : 4])
+  {
+#pragma clang fp contract(off) // a product fused into its first addition would depend on NL
+#pragma unroll
+    for (int s = NL == 32 ? 1 : 2; s >= 1; s >>= 1)
+#pragma unroll
+      for (int i = 0; i < s; ++i) t[i] += t[i + s];
+    double v = t[0];
+    if constexpr (NL == 32) v = dev::pair_sum16(v, v); // bit 4
+    if constexpr (NL >= 16) v += dev::dpp_f64<0x128>(v); // bit 3
+    v += dev::dpp_f64<0xB1>(v);
+    v += dev::dpp_f64<0x4E>(v);
+    v += dev::dpp_f64<0x141>(v);
+    return v;
+  }
+  // The sums of kind 0 and kind 1 of this lane's point, to all its lanes.
+  template <int NL> __device__ __forceinline__ void both_kinds(double v, int kind, double &i0, double &i1)
+  {
+    if constexpr (NL == 8) {
+      const double o = dev::dpp_f64<0x128>(v); // the other eight lanes of the row
+      i0 = kind ? o : v;
+      i1 = kind ? v : o;
+    } else {
+      dev::swap_halves<NL>(v, i0, i1);
+    }
+  }
+
+  // The four stages of one run.  x0: grid point of LDS entry 0; entry p belongs to slot (p - 1) mod SLOTS.
+  template <int NL>
+  __device__ __forceinline__ void flow_stages(const FlowDev &F, const FlowRun &run, int step, double *u_new,
+                                              const double2 *s_nodes, const double *s_exp2, double *s_u,
+                                              double *s_acc, double (*s_y)[kSpan])
+  {
+    constexpr int SLOTS = kRunBlock / (2 * NL), EV = 64 / NL, UN = EV < 4 ? EV : 4;
+    const int tid = threadIdx.x, sub = tid & (NL - 1), kind = (tid / NL) & 1, slot = tid / (2 * NL);
+    const int n = run.n, a = run.a, b = run.b, x0 = a - kHalo - 1;
+    const double dt = F.dt;
+    const Bose B(run.T);
+    const double k_t = F.kt[3 * step], k_half = F.kt[3 * step + 1], k_dt = F.kt[3 * step + 2];
+    // up to four nodes per lane stay in registers
+    constexpr bool KEEP = EV <= 4;
+    double2 kept[KEEP ? EV : 1];
+    if (KEEP)
+#pragma unroll
+      for (int i = 0; i < (KEEP ? EV : 1); ++i) kept[i] = s_nodes[sub + NL * i];
+    for (int stage = 1; stage <= 4; ++stage) {
+      const int w = 4 - stage;
+      const int p0 = max(a - w, 0) - x0, p1 = min(b + w, n) - x0; // evaluated entries [p0, p1)
+      const double k = stage == 1 ? k_t : (stage == 4 ? k_dt : k_half);
+      const double k2 = k * k, k5 = k2 * k2 * k;
+      const double *y = stage == 1 ? s_u : s_y[stage & 1];
+      double *y_next = s_y[(stage & 1) ^ 1];
+      for (int p = 1 + slot; p < p1; p += SLOTS) {
+        if (p < p0) continue;
+        // second-order stencils; at a grid end the neighbours of the next point inside, with the
+        // one-sided first derivative (d -+ 2 dd)/(2h)
+        const int x = x0 + p, in = x == 0 ? 1 : x == n - 1 ? -1 : 0;
+        const double yv = y[p], yl = y[p + in - 1], yc = y[p + in], yr = y[p + in + 1];
+        const double dd = (yr - 2.0 * yc) + yl;
+        const double up = fma(-2.0 * in, dd, yr - yl) * run.i2h, upp = dd * run.ih2;
+        const double rho2 = 2.0 * (x * run.h);
+        const double m2 = kind ? fma(rho2, up, yv) : yv;
+        double v = 0.0;
+        for (int c = 0; c < F.nx; c += 64) {
+          // four nodes at a time; the second four of NL = 8 add bit 5
+          double t[UN];
+#pragma unroll 1
+          for (int g = 0; g < EV; g += UN)
+#pragma unroll
+            for (int i = 0; i < UN; ++i) {
+              const double2 nd = KEEP && c == 0 ? kept[KEEP ? i : 0] : s_nodes[c + sub + NL * (g + i)];
+              const double e = nd.y * bose_4S2(fma(k2, nd.x, m2), B, s_exp2);
+              t[i] = g == 0 ? e : add_plain(t[i], e);
+            }
+          v += node_tree<NL>(t);
+        }
+        double i0, i1;
+        both_kinds<NL>(v, kind, i0, i1);
+        const double f = 0.5 * k5 * ((run.N - 1.0) * up * i0 + (3.0 * up + rho2 * upp) * i1);
+        // the RK4 stage update, by the point's first lane
+        if (kind == 0 && sub == 0) {
+          const double u = s_u[p];
+          if (stage == 1) {
+            s_acc[p] = f;
+            y_next[p] = u + 0.5 * dt * f;
+          } else if (stage < 4) {
+            s_acc[p] += 2.0 * f;
+            y_next[p] = u + (stage == 2 ? 0.5 * dt : dt) * f;
+          } else {
+            const double un = u + dt / 6.0 * (s_acc[p] + f);
+            u_new[x] = un;
+            if (!isfinite(un)) atomicOr(&F.bad[run.slot], 1);
+          }
+        }
+      }
+      __syncthreads();
+    }
   }
 
   // One RK4 step of every resident flow.  A workgroup takes a run [a, b) of one flow and keeps the
@@ -98,137 +238,46 @@ namespace
   // previous stage's values at their neighbours, which the previous stage computed on a range one
   // point wider: points outside the run are evaluated again by the workgroup that owns them, with
   // the same inputs and arithmetic, so every point's result is what a stage-by-stage sweep gives
-  // and does not depend on how flows are cut into runs.  Within a stage the waves share the points
-  // two at a time (lanes over Gauss-Legendre nodes).  u is read from the buffer of this step's
+  // and does not depend on how flows are cut into runs.  u is read from the buffer of this step's
   // parity and written to the other, so neighbouring runs read the old u.
-  __global__ __launch_bounds__(kRunBlock) void flow_step_kernel(FlowDev F, int local)
+  //
+  // What bounds it: VALU issue when the runs fill the CUs, the dependent chain of a stage (stencil,
+  // nodes, reduction, update, barrier) when they do not.  So a point's two integrals sit in
+  // neighbouring lanes that also form its stencil and its update (one barrier per stage, no hand-over
+  // through LDS but the stage's value), eight lanes each, so that a lane has eight independent nodes in
+  // flight and the reduction is three steps; short runs spread a point over 16 or 32 lanes.  With a
+  // node per lane, 64-lane reductions and three barriers a step of 13,054 points took 22.2 us, of one
+  // 64-point flow 9.4; now 16.7 and 6.2.
+  __global__ __launch_bounds__(kRunBlock, 4) void flow_step_kernel(FlowDev F, int local)
   {
-    __shared__ double s_exp2[64]; // 2^(j/64)
-    __shared__ double s_u[kSpan], s_y[kSpan], s_acc[kSpan], s_f[kSpan];
-    __shared__ double s_m2pi[kSpan], s_m2sig[kSpan], s_up[kSpan], s_upp[kSpan];
-    for (int j = threadIdx.x; j < 64; j += kRunBlock) s_exp2[j] = exp2(j * (1.0 / 64.0));
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int n_wv = kRunBlock / 64;
-    const int R = *F.n_runs;
-    const int base = *F.base + local;
-    // node factors, one node per lane when there are at most 64 (the rest loop over nodes)
-    const bool lane_nodes = F.nx <= 64;
-    double A_l = 0.0, D_l = 0.0;
-    if (lane_nodes && lane < F.nx) {
-      A_l = F.A[lane];
-      D_l = F.D[lane];
-    }
-    __syncthreads();
+    extern __shared__ double2 s_nodes[]; // F.nodes
+    __shared__ double s_exp2[kFlowExp];
+    __shared__ double s_u[kSpan], s_acc[kSpan], s_y[2][kSpan];
+    const int tid = threadIdx.x;
+    const int R = *F.n_runs, base = *F.base + local;
+    // the first run's record is loaded beside the count (the table has kMaxFlowGrid entries at least)
+    if (F.runs[blockIdx.x].n == 0 || (int)blockIdx.x >= R) return;
+    for (int j = tid; j < (F.nx + 63) / 64 * 64; j += kRunBlock) s_nodes[j] = F.nodes[j];
+    for (int j = tid; j < kFlowExp; j += kRunBlock) s_exp2[j] = F.exp2t[j];
     for (int r = blockIdx.x; r < R; r += gridDim.x) {
       const FlowRun run = F.runs[r]; // workgroup-uniform
       const int step = base - run.admit;
-      // a flow outside its steps, or idle, is left alone (workgroup-uniform)
-      if (step < 0 || step >= F.n_steps || F.status[run.slot] != 1) continue;
-      const int n = run.n, a = run.a, b = run.b;
-      const double h = F.h[run.slot], T = F.T[run.slot], Nn = F.N[run.slot], dt = F.dt;
-      const double k_t = F.kt[3 * step], k_half = F.kt[3 * step + 1], k_dt = F.kt[3 * step + 2];
-      const double inv_T = 1.0 / T, inv_8T = 0.125 * inv_T;
+      if (step < 0 || step >= F.n_steps) continue; // outside its steps (workgroup-uniform)
+      const int n = run.n, len = run.b - run.a, x0 = run.a - kHalo - 1;
       const double *u_old = F.pool + run.off + (step & 1) * n;
       double *u_new = F.pool + run.off + ((step + 1) & 1) * n;
-      const int x0 = a - kHalo - 1; // grid point of LDS entry 0
       // step 0 starts from the initial condition itself, so admission copies nothing to the device
-      const bool initial = step == 0;
-      const double m2_0 = F.m2_0[run.slot], half_lam = 0.5 * F.lam[run.slot];
-      for (int i = tid; i < b - a + 2 * (kHalo + 1); i += kRunBlock) {
+      for (int i = tid; i < len + 2 * (kHalo + 1); i += kRunBlock) {
         const int x = x0 + i;
-        const double v = x >= 0 && x < n ? (initial ? m2_0 + half_lam * (x * h) : u_old[x]) : 0.0;
-        s_u[i] = v;
-        s_y[i] = v;
+        s_u[i] = x >= 0 && x < n ? (step == 0 ? run.m2_0 + 0.5 * run.lam * (x * run.h) : u_old[x]) : 0.0;
       }
       __syncthreads();
-      for (int stage = 1; stage <= 4; ++stage) {
-        const int w = 4 - stage;
-        const int p0 = max(a - w, 0) - x0, p1 = min(b + w, n) - x0; // evaluated entries [p0, p1)
-        const double k = stage == 1 ? k_t : (stage == 4 ? k_dt : k_half);
-        // stencil terms of the evaluated points from this stage's input
-        for (int p = p0 + tid; p < p1; p += kRunBlock) {
-          const int x = x0 + p;
-          const double yv = s_y[p];
-          double up, upp;
-          if (x == 0) {
-            up = (-3.0 * yv + 4.0 * s_y[p + 1] - s_y[p + 2]) / (2.0 * h);
-            upp = (yv - 2.0 * s_y[p + 1] + s_y[p + 2]) / (h * h);
-          } else if (x == n - 1) {
-            up = (3.0 * yv - 4.0 * s_y[p - 1] + s_y[p - 2]) / (2.0 * h);
-            upp = (yv - 2.0 * s_y[p - 1] + s_y[p - 2]) / (h * h);
-          } else {
-            up = (s_y[p + 1] - s_y[p - 1]) / (2.0 * h);
-            upp = (s_y[p + 1] - 2.0 * yv + s_y[p - 1]) / (h * h);
-          }
-          const double rho = x * h;
-          s_up[p] = up;
-          s_upp[p] = upp;
-          s_m2pi[p] = yv;
-          s_m2sig[p] = yv + 2.0 * rho * up;
-        }
-        __syncthreads();
-        // right-hand sides, two points per wave at a time: their four node sums (two threshold
-        // integrals each) are reduced together by dev::wave_sum4 (kind of point pp: vector 2 pp + kind)
-        const double k2 = k * k, k5 = k * k * (k * k) * k;
-        for (int g0 = p0 + kGroup * wave; g0 < p1; g0 += kGroup * n_wv) {
-          double v[2 * kGroup];
-#pragma unroll
-          for (int pp = 0; pp < kGroup; ++pp) {
-            const int p = g0 + pp;
-            double ipi = 0.0, isg = 0.0;
-            if (p < p1) { // wave-uniform
-              const double pm2pi = s_m2pi[p], pm2sig = s_m2sig[p];
-              // two threshold integrals, lane j evaluates node j (d = 3 radial element)
-              if (lane_nodes) {
-                if (lane < F.nx) {
-                  ipi = fma(D_l, bose_S2(fma(k2, A_l, pm2pi), T, inv_8T, inv_T, s_exp2), 0.0);
-                  isg = fma(D_l, bose_S2(fma(k2, A_l, pm2sig), T, inv_8T, inv_T, s_exp2), 0.0);
-                }
-              } else {
-                for (int j = lane; j < F.nx; j += 64) {
-                  const double an = F.A[j], dd = F.D[j];
-                  ipi = fma(dd, bose_S2(fma(k2, an, pm2pi), T, inv_8T, inv_T, s_exp2), ipi);
-                  isg = fma(dd, bose_S2(fma(k2, an, pm2sig), T, inv_8T, inv_T, s_exp2), isg);
-                }
-              }
-            }
-            v[2 * pp] = ipi;
-            v[2 * pp + 1] = isg;
-          }
-          const double sum = dev::wave_sum4(v);
-#pragma unroll
-          for (int pp = 0; pp < kGroup; ++pp) {
-            const int p = g0 + pp;
-            if (p >= p1) continue; // wave-uniform
-            const double ipi = k5 * dev::lane_value(sum, dev::sum8_lane(2 * pp));
-            const double isg = k5 * dev::lane_value(sum, dev::sum8_lane(2 * pp + 1));
-            if (lane == 0) {
-              const double up = s_up[p], upp = s_upp[p], rho = (x0 + p) * h;
-              s_f[p] = 0.5 * ((Nn - 1.0) * up * ipi + (3.0 * up + 2.0 * rho * upp) * isg);
-            }
-          }
-        }
-        __syncthreads();
-        // the RK4 stage update of the evaluated points
-        for (int p = p0 + tid; p < p1; p += kRunBlock) {
-          const double f = s_f[p], u = s_u[p];
-          if (stage == 1) {
-            s_acc[p] = f;
-            s_y[p] = u + 0.5 * dt * f;
-          } else if (stage == 2) {
-            s_acc[p] = s_acc[p] + 2.0 * f;
-            s_y[p] = u + 0.5 * dt * f;
-          } else if (stage == 3) {
-            s_acc[p] = s_acc[p] + 2.0 * f;
-            s_y[p] = u + dt * f;
-          } else {
-            const double un = u + dt / 6.0 * (s_acc[p] + f);
-            u_new[x0 + p] = un;
-            if (!isfinite(un)) atomicOr(&F.bad[run.slot], 1);
-          }
-        }
-        __syncthreads();
-      }
+      if (len + 2 * kHalo <= kRunBlock / 64) // 16 points
+        flow_stages<32>(F, run, step, u_new, s_nodes, s_exp2, s_u, s_acc, s_y);
+      else if (len + 2 * kHalo <= kRunBlock / 32)
+        flow_stages<16>(F, run, step, u_new, s_nodes, s_exp2, s_u, s_acc, s_y);
+      else
+        flow_stages<8>(F, run, step, u_new, s_nodes, s_exp2, s_u, s_acc, s_y);
     }
   }
 
@@ -252,11 +301,11 @@ struct FlowRecord {
   std::vector<double> u;
 };
 
-// The per-slot parameters and the run count live in one device block with a pinned host mirror:
-// the host edits the mirror and uploads it with one asynchronous copy before a launch, and the
+// The per-slot flags and the run count live in one device block with a pinned host mirror: the
+// host edits the mirror and uploads it with one asynchronous copy before a launch, and the
 // launch's non-finite flags come back into the mirror behind the graph.
 struct SlotLayout {
-  size_t n_runs = 0, status = 0, bad = 0, h = 0, T = 0, N = 0, m2_0 = 0, lam = 0, bytes = 0;
+  size_t n_runs = 0, bad = 0, bytes = 0;
 };
 
 struct dfrg_fs {
@@ -273,10 +322,10 @@ struct dfrg_fs {
   bool runs_dirty = true;
   size_t runs_cap = 0; // FlowRun entries allocated on the device
   hipStream_t stream = nullptr;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t graph_exec = nullptr;
+  hipGraph_t graph[kFlowGraphs] = {};
+  hipGraphExec_t graph_exec[kFlowGraphs] = {};
   int base = 0;           // global step index of the next launch's first step (mirrors dev.base)
-  double *d_nodes = nullptr; // A | D | kt
+  double *d_nodes = nullptr; // (A, D/4) | 2^(j/512) | kt
   std::vector<double> latencies;
   double busy_s = 0;
   int finished = 0;
@@ -330,24 +379,33 @@ namespace
     fs->free_ranges.swap(merged);
   }
 
-  int fs_capture(dfrg_fs *fs)
+  // The graph of steps_per_launch steps with the smallest power-of-two grid (64 to kMaxFlowGrid) of at
+  // least the resident runs: workgroups without a run would still be dispatched.  Each is captured
+  // once, when first needed.
+  int fs_capture(dfrg_fs *fs, hipGraphExec_t *exec)
   {
-    if (fs->graph_exec) return DFRG_OK;
+    const int R = *fs->mirror<int>(fs->sl.n_runs);
+    int g = 0;
+    while ((64 << g) < R && (64 << g) < kMaxFlowGrid) ++g;
+    *exec = fs->graph_exec[g];
+    if (*exec) return DFRG_OK;
     hipStream_t cs;
     DFRG_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
     DFRG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
+    const size_t shm = sizeof(double2) * ((fs->nx + 63) / 64 * 64);
     for (int st = 0; st < fs->steps_per_launch; ++st)
-      hipLaunchKernelGGL(flow_step_kernel, dim3(kFlowGrid), dim3(kRunBlock), 0, cs, fs->dev, st);
+      hipLaunchKernelGGL(flow_step_kernel, dim3(64 << g), dim3(kRunBlock), shm, cs, fs->dev, st);
     hipLaunchKernelGGL(flow_base_kernel, dim3(1), dim3(64), 0, cs, fs->dev.base, fs->steps_per_launch);
-    hipGraph_t g = nullptr;
-    hipError_t e = hipStreamEndCapture(cs, &g);
+    hipGraph_t gr = nullptr;
+    hipError_t e = hipStreamEndCapture(cs, &gr);
     hipStreamDestroy(cs);
     if (e != hipSuccess) {
       set_error("flow graph capture failed: %s", hipGetErrorString(e));
       return DFRG_ERR_HIP;
     }
-    fs->graph = g;
-    DFRG_HIP(hipGraphInstantiate(&fs->graph_exec, g, nullptr, nullptr, 0));
+    fs->graph[g] = gr;
+    DFRG_HIP(hipGraphInstantiate(&fs->graph_exec[g], gr, nullptr, nullptr, 0));
+    *exec = fs->graph_exec[g];
     return DFRG_OK;
   }
 
@@ -381,8 +439,6 @@ namespace
         ++fs->finished;
       }
       fs_free_range(fs, r.off, 2 * n);
-      fs->mirror<int>(fs->sl.status)[s] = 0;
-      fs->slots_dirty = true;
       fs->slot_flow[s] = -1;
       r.slot = -1;
       fs->runs_dirty = true;
@@ -406,16 +462,9 @@ namespace
       const int off = fs_alloc_range(fs, 2 * n);
       if (off < 0) break; // does not fit the HBM budget now: wait for retirements (FIFO)
       fs->queue.pop_front();
-      // the slot's parameters go to the mirror; step 0 reads the initial condition from them, and
-      // writes the odd buffer, so the flow's HBM range needs no initialisation
-      const SlotLayout &L = fs->sl;
-      fs->mirror<int>(L.status)[slot] = 1;
-      fs->mirror<int>(L.bad)[slot] = 0;
-      fs->mirror<double>(L.h)[slot] = r.desc.rho_max / (n - 1);
-      fs->mirror<double>(L.T)[slot] = r.desc.T;
-      fs->mirror<double>(L.N)[slot] = r.desc.N;
-      fs->mirror<double>(L.m2_0)[slot] = r.desc.m2_0;
-      fs->mirror<double>(L.lam)[slot] = r.desc.lambda;
+      // step 0 reads the initial condition from the run records, and writes the odd buffer, so the
+      // flow's HBM range needs no initialisation
+      fs->mirror<int>(fs->sl.bad)[slot] = 0;
       fs->slots_dirty = true;
       fs->slot_flow[slot] = id;
       r.slot = slot;
@@ -425,32 +474,41 @@ namespace
       fs->runs_dirty = true;
     }
     if (fs->runs_dirty) {
-      // cut every resident flow into runs of at most L points, with the smallest L (>= 8) whose
-      // runs fit the workgroups resident at once (two per CU), so that a step takes one round of
-      // workgroups (a flow of n >= 4 points then has runs of >= 2 points)
+      // cut every resident flow into runs of at most L points (and at least 2).  A workgroup holds 64
+      // points of a stage at eight lanes per integral, 32 or 16 at 16 or 32, and a run's first stage
+      // has L + 6; the L whose step is cheapest: per round of one workgroup on each CU a fixed part (its
+      // first loads, about 250 instruction slots a stage) and the VALU instructions of a SIMD's waves
+      // (155, 220 and 350 per stage for waves of one, two and four points)
       std::vector<int> sizes;
-      long long P = 0;
       for (int s = 0; s < fs->max_resident; ++s)
-        if (fs->slot_flow[s] >= 0) {
-          sizes.push_back(fs->flows[fs->slot_flow[s]].desc.n_grid);
-          P += sizes.back();
-        }
-      const long long slots = 2LL * (context().cu_count > 0 ? context().cu_count : 256);
-      int L = (int)std::min<long long>(kMaxRun, std::max<long long>(8, (P + slots - 1) / slots));
-      auto count = [&](int len) {
+        if (fs->slot_flow[s] >= 0) sizes.push_back(fs->flows[fs->slot_flow[s]].desc.n_grid);
+      const long long cus = context().cu_count > 0 ? context().cu_count : 256;
+      auto pieces = [](int n, int len) { return std::min((n + len - 1) / len, n / 2); };
+      int L = kMaxRun;
+      double best = 1e300;
+      for (int len : kRunLengths) {
         long long c = 0;
-        for (int n : sizes) c += (n + len - 1) / len;
-        return c;
-      };
-      while (L < kMaxRun && count(L) > slots) ++L;
+        for (int n : sizes) c += pieces(n, len);
+        const int first = len + 2 * kHalo;
+        const int issue = first <= 16   ? (first + 3) / 4 * 155
+                          : first <= 32 ? (first + 7) / 8 * 220
+                                        : (first + 15) / 16 * 350;
+        const double cost = (double)((c + cus - 1) / cus) * (250 + issue);
+        if (cost < best) {
+          best = cost;
+          L = len;
+        }
+      }
       std::vector<FlowRun> runs;
       for (int s = 0; s < fs->max_resident; ++s) {
         if (fs->slot_flow[s] < 0) continue;
         const FlowRecord &r = fs->flows[fs->slot_flow[s]];
-        const int n = r.desc.n_grid, cnt = (n + L - 1) / L, len = n / cnt, extra = n % cnt;
+        const int n = r.desc.n_grid, cnt = pieces(n, L), len = n / cnt, extra = n % cnt;
+        const double h = r.desc.rho_max / (n - 1);
         for (int j = 0, a = 0; j < cnt; ++j) {
           const int b = a + len + (j < extra ? 1 : 0);
-          runs.push_back(FlowRun{s, a, b, n, r.off, r.admit});
+          runs.push_back(FlowRun{s, a, b, n, r.off, r.admit, h, 0.5 / h, 1.0 / (h * h), r.desc.T, r.desc.N,
+                                 r.desc.m2_0, r.desc.lambda});
           a = b;
         }
       }
@@ -533,21 +591,26 @@ int dfrg_fs_create(dfrg_fs **out, dfrg_qp *qp, size_t hbm_budget, int max_reside
   }
   // node factors and k(t) (header comment); k as the oracle's stepper forms it: t = s dt,
   // exp(-t), exp(-(t + dt/2)), exp(-(t + dt))
-  std::vector<double> nodes(2 * nx + 3 * (size_t)n_steps);
+  const int nxp = (nx + 63) / 64 * 64;
+  std::vector<double> nodes(2 * nxp + kFlowExp + 3 * (size_t)n_steps);
   for (int j = 0; j < nx; ++j) {
     const double xr = ((const double *)hx)[j] * fs->x_extent;
     const double e = std::exp(-xr);
-    nodes[j] = xr + e;
-    nodes[nx + j] = std::sqrt(xr) * (((const double *)hw)[j] * fs->x_extent) * e * (1.0 + xr) / (2.0 * kPi * kPi);
+    nodes[2 * j] = xr + e;
+    nodes[2 * j + 1] =
+        0.25 * (std::sqrt(xr) * (((const double *)hw)[j] * fs->x_extent) * e * (1.0 + xr) / (2.0 * kPi * kPi));
   }
+  for (int j = nx; j < nxp; ++j) nodes[2 * j] = 1e30;
+  for (int j = 0; j < kFlowExp; ++j) nodes[2 * nxp + j] = (double)std::exp2((long double)j / kFlowExp);
+  double *kt = &nodes[2 * nxp + kFlowExp];
   for (int st = 0; st < n_steps; ++st) {
     const double t = st * d.dt;
-    nodes[2 * nx + 3 * st] = std::exp(-t);
-    nodes[2 * nx + 3 * st + 1] = std::exp(-(t + 0.5 * d.dt));
-    nodes[2 * nx + 3 * st + 2] = std::exp(-(t + d.dt));
+    kt[3 * st] = std::exp(-t);
+    kt[3 * st + 1] = std::exp(-(t + 0.5 * d.dt));
+    kt[3 * st + 2] = std::exp(-(t + d.dt));
   }
-  // runs: at most one per 4 points of each resident flow (n >= 4, L >= 8), plus one per flow
-  fs->runs_cap = std::min(max_points, fs->pool_doubles / 4 + (size_t)max_resident + 1);
+  // runs: at least 2 points each, and a resident flow of n points holds 2 n doubles of the pool
+  fs->runs_cap = std::max<size_t>(std::min(max_points, fs->pool_doubles / 4 + (size_t)max_resident + 1), kMaxFlowGrid);
   const size_t runs_bytes = sizeof(FlowRun) * fs->runs_cap;
 #define FS_ALLOC(ptr, bytes)                                                                                   \
   do {                                                                                                         \
@@ -563,13 +626,7 @@ int dfrg_fs_create(dfrg_fs **out, dfrg_qp *qp, size_t hbm_budget, int max_reside
     const size_t M = (size_t)max_resident;
     size_t o = 0;
     L.n_runs = o, o += up(sizeof(int));
-    L.status = o, o += up(sizeof(int) * M);
     L.bad = o, o += up(sizeof(int) * M);
-    L.h = o, o += up(sizeof(double) * M);
-    L.T = o, o += up(sizeof(double) * M);
-    L.N = o, o += up(sizeof(double) * M);
-    L.m2_0 = o, o += up(sizeof(double) * M);
-    L.lam = o, o += up(sizeof(double) * M);
     L.bytes = o;
   }
   FS_ALLOC(fs->d_slots, fs->sl.bytes);
@@ -581,21 +638,15 @@ int dfrg_fs_create(dfrg_fs **out, dfrg_qp *qp, size_t hbm_budget, int max_reside
   }
   std::memset(fs->h_slots, 0, fs->sl.bytes);
   d.n_runs = (int *)(fs->d_slots + fs->sl.n_runs);
-  d.status = (int *)(fs->d_slots + fs->sl.status);
   d.bad = (int *)(fs->d_slots + fs->sl.bad);
-  d.h = (double *)(fs->d_slots + fs->sl.h);
-  d.T = (double *)(fs->d_slots + fs->sl.T);
-  d.N = (double *)(fs->d_slots + fs->sl.N);
-  d.m2_0 = (double *)(fs->d_slots + fs->sl.m2_0);
-  d.lam = (double *)(fs->d_slots + fs->sl.lam);
   FS_ALLOC(d.runs, runs_bytes);
   FS_ALLOC(d.base, sizeof(int));
   FS_ALLOC(fs->d_nodes, sizeof(double) * nodes.size());
   FS_ALLOC(d.pool, sizeof(double) * fs->pool_doubles);
 #undef FS_ALLOC
-  d.A = fs->d_nodes;
-  d.D = fs->d_nodes + nx;
-  d.kt = fs->d_nodes + 2 * nx;
+  d.nodes = (const double2 *)fs->d_nodes;
+  d.exp2t = fs->d_nodes + 2 * nxp;
+  d.kt = fs->d_nodes + 2 * nxp + kFlowExp;
   if (hipMemcpy(fs->d_nodes, nodes.data(), sizeof(double) * nodes.size(), hipMemcpyHostToDevice) != hipSuccess) {
     set_error("flow server: node table upload failed");
     dfrg_fs_destroy(fs);
@@ -616,8 +667,10 @@ int dfrg_fs_destroy(dfrg_fs *fs)
 {
   if (!fs) return DFRG_OK;
   hipDeviceSynchronize();
-  if (fs->graph_exec) hipGraphExecDestroy(fs->graph_exec);
-  if (fs->graph) hipGraphDestroy(fs->graph);
+  for (int g = 0; g < kFlowGraphs; ++g) {
+    if (fs->graph_exec[g]) hipGraphExecDestroy(fs->graph_exec[g]);
+    if (fs->graph[g]) hipGraphDestroy(fs->graph[g]);
+  }
   if (fs->ev0) hipEventDestroy(fs->ev0);
   if (fs->ev1) hipEventDestroy(fs->ev1);
   if (fs->stream) hipStreamDestroy(fs->stream);
@@ -655,7 +708,8 @@ int dfrg_fs_progress(dfrg_fs *fs, int *resident, int *queued, int *done)
   DFRG_CHECK_ARG(fs != nullptr, "NULL server");
   DFRG_TRY(fs_admit(fs));
   if (resident_count(fs) > 0) {
-    DFRG_TRY(fs_capture(fs));
+    hipGraphExec_t graph = nullptr;
+    DFRG_TRY(fs_capture(fs, &graph));
     // grid-point steps this launch advances: each resident flow takes the steps it has left, up to
     // steps_per_launch
     for (long long id : fs->slot_flow)
@@ -691,7 +745,7 @@ int dfrg_fs_progress(dfrg_fs *fs, int *resident, int *queued, int *done)
                               fs->stream));
     fs->runs_upload = 0;
     DFRG_HIP(hipEventRecord(fs->ev0, fs->stream));
-    DFRG_HIP(hipGraphLaunch(fs->graph_exec, fs->stream));
+    DFRG_HIP(hipGraphLaunch(graph, fs->stream));
     DFRG_HIP(hipEventRecord(fs->ev1, fs->stream));
     // behind the graph: the non-finite flags into the mirror, and the finishers' final u
     DFRG_HIP(hipMemcpyAsync(fs->h_slots + fs->sl.bad, fs->dev.bad, sizeof(int) * fs->max_resident,

@@ -71,6 +71,25 @@ namespace dfrg
       const double b2 = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
       return a2 + b2;
     }
+    // Neighbouring groups of N lanes (N = 16: the rows of a 32-lane half, N = 32: the halves of the wave):
+    // `first` gets the first group's v in both, `second` the second group's.
+    template <int N> __device__ __forceinline__ void swap_halves(double v, double &first, double &second)
+    {
+      const unsigned long long u = __double_as_longlong(v);
+      const unsigned l = (unsigned)u, h = (unsigned)(u >> 32);
+      if constexpr (N == 32) {
+        const auto lo = __builtin_amdgcn_permlane32_swap(l, l, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(h, h, false, false);
+        first = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+        second = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+      } else {
+        static_assert(N == 16);
+        const auto lo = __builtin_amdgcn_permlane16_swap(l, l, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+        first = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+        second = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+      }
+    }
     __device__ __forceinline__ double wave_sum8(const double (&v)[8])
     {
       const double w0 = pair_sum32(v[0], v[1]), w1 = pair_sum32(v[2], v[3]);
