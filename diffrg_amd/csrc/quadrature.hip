@@ -174,8 +174,8 @@ namespace dfrg
     // One wave per node: every block forms the matrix in its LDS.  Rounds of 64 points shrink the bracket
     // about 64-fold each, nine quick counts and two with pivots against 70 bisection steps with pivots,
     // whose division chain bounded the kernel (all nodes had shared one block); the two halves of the
-    // twisted factorisation run on two lanes.  A call for 66 nodes, launch to synchronised
-    // result, 414 -> 87 us, for 32 nodes 213 -> 75, most of what is left on the host.
+    // twisted factorisation run on two lanes.  A provider's rule
+    // of 66 nodes, call to result, 414 -> 50 us, of 32 nodes 213 -> 39.
     __global__ __launch_bounds__(64) void matsubara_kernel(int n, double T, double *x_out, double *w_out)
     {
       extern __shared__ double sm[];
@@ -305,10 +305,16 @@ namespace dfrg
       w[i + h] = (gw[i] * log_ext * xl) / two_pi;
     }
 
-    __global__ void to_f32_kernel(int n, const double *a, float *b)
+    // FP32 copies of a rule, and its host copies in pinned staging, behind the kernel that made it
+    __global__ void rule_copies_kernel(int n, const double *x, const double *w, float *xf, float *wf, double *h)
     {
       const int i = blockIdx.x * blockDim.x + threadIdx.x;
-      if (i < n) b[i] = (float)a[i];
+      if (i >= n) return;
+      const double xi = x[i], wi = w[i];
+      xf[i] = (float)xi;
+      wf[i] = (float)wi;
+      h[i] = xi;
+      h[n + i] = wi;
     }
 
     // LDS of gl_kernel: the reciprocals of 1..order (64 KB at 4096, the largest order)
@@ -335,6 +341,46 @@ namespace dfrg
 
 using namespace dfrg;
 
+namespace
+{
+  // dfrg_matsubara_generate without its synchronisation
+  int enqueue_matsubara(double T, double E, int step, int min_size, int max_size, int vacuum_quad_size,
+                        int precision_factor, double *d_x, double *d_w, int cap, int *size, double *T_rule,
+                        hipStream_t s)
+  {
+    DFRG_CHECK_ARG(step >= 1, "step must be positive");
+    DFRG_CHECK_ARG(std::isfinite(T) && std::isfinite(E) && T >= 0.0, "invalid T=%g / E=%g", T, E);
+    if (precision_factor < 0) precision_factor = 1;
+    if (vacuum_quad_size <= 6) vacuum_quad_size = 6;
+    int m = predict_size(T, E, step, vacuum_quad_size, precision_factor);
+    if (m < 0) {
+      m = -m;
+      if (m % 2) ++m;
+      DFRG_CHECK_ARG(m <= cap, "vacuum Matsubara rule of %d nodes exceeds capacity %d", m, cap);
+      if (is_close_abs(E, 0.0, 2.220446049250313e-16)) E = 1.0;
+      const int h = m / 2;
+      double *g = nullptr;
+      DFRG_HIP(hipMallocAsync((void **)&g, sizeof(double) * 2 * h, s));
+      hipLaunchKernelGGL(gl_kernel, dim3((h + 1) / 2 / kGlBlock + 1), dim3(kGlBlock), gl_shared(h), s, h, g, g + h);
+      DFRG_LAUNCHED("gl_kernel");
+      hipLaunchKernelGGL(matsubara_vacuum_kernel, dim3(h / 64 + 1), dim3(64), 0, s, h, E, g, g + h, d_x, d_w);
+      DFRG_LAUNCHED("matsubara_vacuum_kernel");
+      DFRG_HIP(hipFreeAsync(g, s));
+      *size = m;
+      if (T_rule) *T_rule = 0.0;
+      return DFRG_OK;
+    }
+    m = std::max(min_size, std::min(max_size, m));
+    DFRG_CHECK_ARG(m >= 1 && m <= 1024, "Matsubara rule size %d out of range [1,1024]", m);
+    DFRG_CHECK_ARG(m <= cap, "Matsubara rule of %d nodes exceeds capacity %d", m, cap);
+    hipLaunchKernelGGL(matsubara_kernel, dim3(m), dim3(64), 5 * m * sizeof(double), s, m, T, d_x, d_w);
+    DFRG_LAUNCHED("matsubara_kernel");
+    *size = m;
+    if (T_rule) *T_rule = T;
+    return DFRG_OK;
+  }
+} // namespace
+
 extern "C" {
 
 int dfrg_gl_generate(int order, double *d_x, double *d_w, void *stream)
@@ -355,38 +401,10 @@ int dfrg_matsubara_generate(double T, double E, int step, int min_size, int max_
 {
   DFRG_TRY(require_init());
   DFRG_CHECK_ARG(d_x && d_w && size, "output pointers are NULL");
-  DFRG_CHECK_ARG(step >= 1, "step must be positive");
-  DFRG_CHECK_ARG(std::isfinite(T) && std::isfinite(E) && T >= 0.0, "invalid T=%g / E=%g", T, E);
-  if (precision_factor < 0) precision_factor = 1;
-  if (vacuum_quad_size <= 6) vacuum_quad_size = 6;
   hipStream_t s = resolve_stream(stream);
-  int m = predict_size(T, E, step, vacuum_quad_size, precision_factor);
-  if (m < 0) {
-    m = -m;
-    if (m % 2) ++m;
-    DFRG_CHECK_ARG(m <= cap, "vacuum Matsubara rule of %d nodes exceeds capacity %d", m, cap);
-    if (is_close_abs(E, 0.0, 2.220446049250313e-16)) E = 1.0;
-    const int h = m / 2;
-    double *g = nullptr;
-    DFRG_HIP(hipMallocAsync((void **)&g, sizeof(double) * 2 * h, s));
-    hipLaunchKernelGGL(gl_kernel, dim3((h + 1) / 2 / kGlBlock + 1), dim3(kGlBlock), gl_shared(h), s, h, g, g + h);
-    DFRG_LAUNCHED("gl_kernel");
-    hipLaunchKernelGGL(matsubara_vacuum_kernel, dim3(h / 64 + 1), dim3(64), 0, s, h, E, g, g + h, d_x, d_w);
-    DFRG_LAUNCHED("matsubara_vacuum_kernel");
-    DFRG_HIP(hipFreeAsync(g, s));
-    DFRG_HIP(hipStreamSynchronize(s));
-    *size = m;
-    if (T_rule) *T_rule = 0.0;
-    return DFRG_OK;
-  }
-  m = std::max(min_size, std::min(max_size, m));
-  DFRG_CHECK_ARG(m >= 1 && m <= 1024, "Matsubara rule size %d out of range [1,1024]", m);
-  DFRG_CHECK_ARG(m <= cap, "Matsubara rule of %d nodes exceeds capacity %d", m, cap);
-  hipLaunchKernelGGL(matsubara_kernel, dim3(m), dim3(64), 5 * m * sizeof(double), s, m, T, d_x, d_w);
-  DFRG_LAUNCHED("matsubara_kernel");
+  DFRG_TRY(enqueue_matsubara(T, E, step, min_size, max_size, vacuum_quad_size, precision_factor, d_x, d_w, cap, size,
+                             T_rule, s));
   DFRG_HIP(hipStreamSynchronize(s));
-  *size = m;
-  if (T_rule) *T_rule = T;
   return DFRG_OK;
 }
 
@@ -406,6 +424,10 @@ struct Rule {
 
 struct dfrg_qp {
   std::mutex mutex;
+  // The rules' device memory: a few large blocks instead of four allocations per rule, given back when
+  // the provider is destroyed.
+  std::vector<char *> slabs;
+  size_t slab_used = 0, slab_cap = 0;
   int vacuum_quad_size = 48;
   int min_matsubara_size = 32;
   int add_matsubara_size = 0;
@@ -415,30 +437,63 @@ struct dfrg_qp {
 
 namespace
 {
-  int finish_rule(Rule &r, hipStream_t s)
+  // Room for a rule of up to cap nodes: x, w (FP64), then their FP32 copies.
+  int place_rule(dfrg_qp *qp, Rule &r, int cap)
   {
-    const int n = r.size;
-    DFRG_HIP(hipMalloc((void **)&r.d_xf, sizeof(float) * n));
-    DFRG_HIP(hipMalloc((void **)&r.d_wf, sizeof(float) * n));
-    hipLaunchKernelGGL(to_f32_kernel, dim3(n / 64 + 1), dim3(64), 0, s, n, r.d_x, r.d_xf);
-    hipLaunchKernelGGL(to_f32_kernel, dim3(n / 64 + 1), dim3(64), 0, s, n, r.d_w, r.d_wf);
-    DFRG_LAUNCHED("to_f32_kernel");
-    r.hx.resize(n);
-    r.hw.resize(n);
-    DFRG_HIP(hipMemcpyAsync(r.hx.data(), r.d_x, sizeof(double) * n, hipMemcpyDeviceToHost, s));
-    DFRG_HIP(hipMemcpyAsync(r.hw.data(), r.d_w, sizeof(double) * n, hipMemcpyDeviceToHost, s));
-    DFRG_HIP(hipStreamSynchronize(s));
-    r.hxf.assign(r.hx.begin(), r.hx.end());
-    r.hwf.assign(r.hw.begin(), r.hw.end());
+    const size_t c = ((size_t)cap + 31) / 32 * 32, need = c * 2 * (sizeof(double) + sizeof(float));
+    if (qp->slabs.empty() || qp->slab_used + need > qp->slab_cap) {
+      const size_t bytes = std::max<size_t>(need, 64 << 10);
+      void *p = nullptr;
+      DFRG_HIP(hipMalloc(&p, bytes));
+      qp->slabs.push_back((char *)p);
+      qp->slab_used = 0;
+      qp->slab_cap = bytes;
+    }
+    char *p = qp->slabs.back() + qp->slab_used;
+    qp->slab_used += need;
+    r.d_x = (double *)p;
+    r.d_w = r.d_x + c;
+    r.d_xf = (float *)(r.d_w + c);
+    r.d_wf = r.d_xf + c;
     return DFRG_OK;
   }
 
-  void free_rule(Rule &r)
+  // Gives the room of the rule placed last back (a rule that could not be made); returns rc.
+  int unplace_rule(dfrg_qp *qp, const Rule &r, int rc)
   {
-    hipFree(r.d_x);
-    hipFree(r.d_w);
-    hipFree(r.d_xf);
-    hipFree(r.d_wf);
+    qp->slab_used = (size_t)((char *)r.d_x - qp->slabs.back());
+    return rc;
+  }
+
+  // The copies of the rule in flight on s, and the wait for it: one kernel, one synchronisation.
+  int finish_rule(Rule &r, hipStream_t s)
+  {
+    const int n = r.size;
+    void *h = nullptr, *dh = nullptr;
+    DFRG_TRY(dfrg_pool_host_alloc(&h, 2 * sizeof(double) * n));
+    auto work = [&]() -> int {
+      DFRG_HIP(hipHostGetDevicePointer(&dh, h, 0));
+      hipLaunchKernelGGL(rule_copies_kernel, dim3((n + 63) / 64), dim3(64), 0, s, n, r.d_x, r.d_w, r.d_xf, r.d_wf,
+                         (double *)dh);
+      DFRG_LAUNCHED("rule_copies_kernel");
+      return DFRG_OK;
+    };
+    int rc = work();
+    // whatever was launched has finished before the staging goes back to its pool
+    const hipError_t e = hipStreamSynchronize(s);
+    if (rc == DFRG_OK && e != hipSuccess) {
+      set_error("quadrature rule: %s", hipGetErrorString(e));
+      rc = DFRG_ERR_HIP;
+    }
+    if (rc == DFRG_OK) {
+      const double *v = (const double *)h;
+      r.hx.assign(v, v + n);
+      r.hw.assign(v + n, v + 2 * n);
+      r.hxf.assign(r.hx.begin(), r.hx.end());
+      r.hwf.assign(r.hw.begin(), r.hw.end());
+    }
+    dfrg_pool_host_free(h);
+    return rc;
   }
 
   void hand_out(const Rule &r, int fp32, const void **d_x, const void **d_w, const void **h_x, const void **h_w)
@@ -485,9 +540,7 @@ int dfrg_qp_destroy(dfrg_qp *qp)
   if (!qp) return DFRG_OK;
   DFRG_TRY(require_init());
   hipDeviceSynchronize();
-  for (auto &kv : qp->gl) free_rule(kv.second);
-  for (auto &t : qp->mats)
-    for (auto &kv : t.second) free_rule(kv.second);
+  for (char *p : qp->slabs) hipFree(p);
   delete qp;
   return DFRG_OK;
 }
@@ -503,11 +556,11 @@ int dfrg_qp_gl(dfrg_qp *qp, int order, int fp32, const void **d_x, const void **
   if (it == qp->gl.end()) {
     Rule r;
     r.size = order;
-    DFRG_HIP(hipMalloc((void **)&r.d_x, sizeof(double) * order));
-    DFRG_HIP(hipMalloc((void **)&r.d_w, sizeof(double) * order));
+    DFRG_TRY(place_rule(qp, r, order));
     hipStream_t s = resolve_stream(nullptr);
-    DFRG_TRY(dfrg_gl_generate(order, r.d_x, r.d_w, s));
-    DFRG_TRY(finish_rule(r, s));
+    int rc = dfrg_gl_generate(order, r.d_x, r.d_w, s);
+    if (rc == DFRG_OK) rc = finish_rule(r, s);
+    if (rc != DFRG_OK) return unplace_rule(qp, r, rc);
     it = qp->gl.emplace(order, std::move(r)).first;
   }
   hand_out(it->second, fp32, d_x, d_w, h_x, h_w);
@@ -528,14 +581,14 @@ int dfrg_qp_matsubara(dfrg_qp *qp, double T, double E, int fp32, int *size, doub
   if (eit == emap.end()) {
     Rule r;
     const int cap = std::max(qp->vacuum_quad_size + 2, 130);
-    DFRG_HIP(hipMalloc((void **)&r.d_x, sizeof(double) * cap));
-    DFRG_HIP(hipMalloc((void **)&r.d_w, sizeof(double) * cap));
+    DFRG_TRY(place_rule(qp, r, cap));
     hipStream_t s = resolve_stream(nullptr);
     // MatsubaraStorage::find_E_d: reinit(T_key, E, 2, min_matsubara_size, 128, vacuum_quad_size,
     // add_matsubara_size) (quadrature_provider.cu:52)
-    DFRG_TRY(dfrg_matsubara_generate(tit->first, E, 2, qp->min_matsubara_size, 128, qp->vacuum_quad_size,
-                                     qp->add_matsubara_size, r.d_x, r.d_w, cap, &r.size, &r.T_rule, s));
-    DFRG_TRY(finish_rule(r, s));
+    int rc = enqueue_matsubara(tit->first, E, 2, qp->min_matsubara_size, 128, qp->vacuum_quad_size,
+                               qp->add_matsubara_size, r.d_x, r.d_w, cap, &r.size, &r.T_rule, s);
+    if (rc == DFRG_OK) rc = finish_rule(r, s);
+    if (rc != DFRG_OK) return unplace_rule(qp, r, rc);
     eit = emap.emplace(E, std::move(r)).first;
   }
   if (size) *size = eit->second.size;
