@@ -8,23 +8,27 @@
 // texture interpolator TexLinearInterpolator1D of the reference.
 //
 // FP64 logarithmic coordinates on the device: the reference's index idx = log1p(u) (N-1)/a,
-// u = (x - c)/b, costs an FP64 division and log1p per call.  Here it comes from a table of sub-cell
-// starts: K sub-cells per cell (K the smallest power of two with |a|/(K(N-1)) <= 1/4), their starts
-// u_m = expm1(a m/(K(N-1))) and 1/(1 + u_m).  An FP32 log2 of the mantissa of 1 + u plus its exponent
-// locates the sub-cell m, and the position in it is
-//   K(N-1)/a log((1 + u)/(1 + u_m)) = K(N-1)/a 2 atanh(z),  z = delta/(2 + delta),
-//   delta = (u - u_m)/(1 + u_m),
-// with the atanh series to z^17 (|z| <= 0.125: truncation below 1e-17); an estimate one sub-cell off
-// (within ~1e-6 of a boundary) is moved by one.  The index agrees with the reference's to its own FP64
-// rounding (~1e-14 of a cell); the clamp to [0, N-1] and the reference's NaN rule (fmax(0, fmin(NaN,
-// N-1)): a NaN index takes the last point) give the ends: u <= -1 takes the first point when
-// -1 <= u and a > 0 (index -inf or negative), the last point otherwise (NaN, or +inf for a < 0);
-// N = 1, bias 0 and NaN bias have a NaN or zero-width index: the last point.  The device code has no
-// branch on the grid, so a user KERNEL's loop-invariant lookups (at q alone) stay hoistable.  Biases
-// beyond +-700 (exp overflows) and grids of more than 2^21 sub-cells per unit of log2 are refused.
+// u = (x - c)/b, costs an FP64 division and log1p per call.  Here it comes from a table of sub-cells:
+// K per cell (K the smallest power of two with |a|/(K(N-1)) <= 1/32), each with the smaller 1 + u_r of its
+// ends.  An FP32 log2 of the mantissa of 1 + u plus its exponent locates the sub-cell m, and
+//   K idx = m + o + K(N-1)/a log1p(delta),  delta = (u - u_r)/(1 + u_r) in [0, 0.0318],
+// o = 0 when the sub-cell's start is the smaller end (a > 0), else 1; log1p as a polynomial of degree 7
+// (Chebyshev interpolation on the sub-cell's range, remainder 7e-17).  An estimate one sub-cell off
+// (within ~1e-5 of a boundary) gives the same sum.  The index agrees with the reference's to its own
+// FP64 rounding (~1e-14 of a cell); the clamp to [0, N-1] and the reference's NaN rule (fmax(0, fmin(NaN,
+// N-1)): a NaN index takes the last point) give the ends: u <= -1 takes the first point when u = -1 and
+// a > 0 (index -inf), the last point otherwise (NaN, or +inf for a < 0); N = 1, bias 0 and NaN bias
+// have a NaN or zero-width index: the last point.  The device code has no branch on the grid, so a
+// user KERNEL's loop-invariant lookups (at q alone) stay hoistable.  Biases beyond +-700 (exp
+// overflows) and grids of more than 2^21 sub-cells per unit of log2 are refused.
+//
+// VALU issue bounds a KERNEL made of lookups, exponentials and divisions: with sub-cells of 1/4, an
+// atanh series to z^17 and the sub-cell corrected by selects, 64 requests of {64, 32, 32} nodes took
+// 33.9 us in the kernel, now 29.7 (155 -> 129 VALU instructions per node).
 #pragma once
 
 #include <cmath>
+#include <limits>
 #include <memory>
 #include <stdexcept>
 #include <type_traits>
@@ -114,14 +118,15 @@ namespace DiFfRG
 
     // the device index of FP64 log coordinates: sub-cell table and constants
     struct LogCells {
-      const double2 *cell = nullptr; // {u_m, 1/(1 + u_m)}, m = 0 .. K(N-1)
-      double c = 0, inv_b = 0;       // u = (x - c) inv_b
-      double two_s = 0, s_ln2 = 0;   // 2 K(N-1)/a, K(N-1)/a ln 2
+      const double2 *cell = nullptr; // {u_r, 1/(1 + u_r)} of sub-cell m = 0 .. K(N-1) - 1
+      double c = 0, inv_b = 0;       // u = (x - c) inv_b; a NaN inv_b sends every point to the last one
+      double s = 0, s_ln2 = 0;       // K(N-1)/a, K(N-1)/a ln 2
+      double off = 0;                // o
       double inv_k = 1;              // 1/K
-      int m_last = 0, k_shift = 0;   // last sub-cell (K(N-1) - 1), log2 K
+      double u_first = 0, u_last = 0; // stand-ins for u = -1 (a > 0: the first point) and for u < -1 or NaN
+      double top = 0;                // N - 1
+      int m_last = 0;                // last sub-cell (K(N-1) - 1)
       int last = 0;                  // last cell (N - 2; 0 for N = 1)
-      int const_last = 0;            // 1: every point takes the last point (N = 1, bias 0 or NaN)
-      int a_pos = 1;                 // bias > 0
     };
 
     void make_cells()
@@ -130,36 +135,41 @@ namespace DiFfRG
       const unsigned N = size;
       LogCells L;
       L.last = N >= 2 ? int(N) - 2 : 0;
+      L.top = N - 1.;
       std::vector<double2> h;
       if (N >= 2 && a == a && a != 0) {
         if (!(std::fabs(a) <= 700.))
           throw std::invalid_argument("LinearInterpolator1D: the bias of LogarithmicCoordinates1D must be within "
                                       "[-700, 700] (exp(bias) overflows beyond)");
         int k_shift = 0;
-        while (std::fabs(a) / ((double)(1u << k_shift) * (N - 1.)) > 0.25) ++k_shift;
+        while (std::fabs(a) / ((double)(1u << k_shift) * (N - 1.)) > 1. / 32) ++k_shift;
         const double K = double(1u << k_shift), subs = K * (N - 1.);
         if (subs / std::fabs(a) * 0.69314718055994530942 > double(1 << 21) || subs > double(1 << 24))
           throw std::invalid_argument("LinearInterpolator1D: too many points for this bias of "
                                       "LogarithmicCoordinates1D (more than 2^21 sub-cells per unit of log2)");
-        h.resize((size_t)subs + 1);
+        h.resize((size_t)subs);
         for (size_t m = 0; m < h.size(); ++m) {
-          const double t = a * (double)m / subs;
-          h[m] = make_double2(std::expm1(t), std::exp(-t));
+          const double t = a * (double)(a > 0 ? m : m + 1) / subs, u = std::expm1(t);
+          h[m] = make_double2(u, a > 0 ? 1. / (1. + u) : std::exp(-t));
         }
         L.c = coordinates.start;
         L.inv_b = 1. / ((coordinates.stop - coordinates.start) / std::expm1(a));
-        L.two_s = 2. * subs / a;
+        L.s = subs / a;
         L.s_ln2 = subs / a * 0.69314718055994530942;
+        L.off = a > 0 ? 0. : 1.;
         L.inv_k = 1. / K;
         L.m_last = int(subs) - 1;
-        L.k_shift = k_shift;
-        L.a_pos = a > 0;
+        L.u_last = a > 0 ? 1e300 : -1. + 0x1p-53;
+        L.u_first = a > 0 ? 0. : L.u_last;
       } else {
         // one point, bias 0 or NaN: the reference's index is 0 x (...)/a with a NaN or infinite
         // factor, or the one point; all points take the last point.  A valid dummy table keeps the
         // device code branch-free.
-        h = {make_double2(0., 1.), make_double2(0., 1.)};
-        L.const_last = 1;
+        h = {make_double2(0., 1.)};
+        L.inv_b = std::numeric_limits<double>::quiet_NaN();
+        L.u_first = L.u_last = 1e300;
+        L.s = 2.;
+        L.inv_k = 1e12;
       }
       void *p = nullptr;
       dfrg::check(dfrg_malloc(&p, sizeof(double2) * h.size()), "LinearInterpolator1D cells");
@@ -173,44 +183,28 @@ namespace DiFfRG
     // the lerp at the reference's index of u = (x - c)/b (device, no branch on the grid)
     __device__ __forceinline__ NT log_cell_lerp(const double u_in) const
     {
-      const bool inside = u_in > -1.; // false for NaN
-      const double u = inside ? u_in : 0.;
+      // u > -1 (false for NaN), or a stand-in beyond the grid's end
+      const double u_first = lc.u_first, u_last = lc.u_last;
+      const double beyond = u_in == -1. ? u_first : u_last;
+      const double u = u_in > -1. ? u_in : beyond;
       // sub-cell estimate: log2(1 + u) = e + log2(mant), mant in [1/2, 1), FP32 log of the mantissa
-      int e = 0;
-      const double mant = frexp(1. + u, &e);
-      const double est = ((double)e + (double)__builtin_amdgcn_logf((float)mant)) * lc.s_ln2;
-      int m = (int)floor(fmax(0., fmin(est, (double)lc.m_last)));
-      const double2 cl = dfrg::gld(lc.cell + m); // {u_m, 1/(1 + u_m)}
+      const double w = 1. + u;
+      const double lg = (double)__builtin_amdgcn_logf((float)__builtin_amdgcn_frexp_mant(w));
+      const double est = ((double)__builtin_amdgcn_frexp_exp(w) + lg) * lc.s_ln2;
+      const int m = (int)fmax(0., fmin(est, (double)lc.m_last));
+      const double2 cl = dfrg::gld(lc.cell + m); // {u_r, 1/(1 + u_r)}
       double dl = (u - cl.x) * cl.y;
-      dl = fmax(-0.5, fmin(dl, 1.0)); // beyond the sub-cell by more than one: the clamp decides
-      // z = dl/(2 + dl): FP32 seed, two FP64 Newton steps
-      const double den = 2. + dl;
-      double r = (double)__builtin_amdgcn_rcpf((float)den);
-      r = fma(r, fma(-den, r, 1.), r);
-      r = fma(r, fma(-den, r, 1.), r);
-      const double z = dl * r, w = z * z;
-      double pz = fma(w, 1. / 17, 1. / 15);
-      pz = fma(pz, w, 1. / 13);
-      pz = fma(pz, w, 1. / 11);
-      pz = fma(pz, w, 1. / 9);
-      pz = fma(pz, w, 1. / 7);
-      pz = fma(pz, w, 1. / 5);
-      pz = fma(pz, w, 1. / 3);
-      pz = fma(pz, w, 1.);
-      double fs = lc.two_s * (z * pz); // position in the sub-cell
-      // the estimate can be one sub-cell off where the index is within ~1e-6 of a boundary
-      const bool down = fs < 0. && m > 0, up = !down && fs >= 1. && m < lc.m_last;
-      m += up ? 1 : down ? -1 : 0;
-      fs += down ? 1. : up ? -1. : 0.;
-      fs = fmax(0., fmin(fs, 1.));
-      // sub-cell -> cell (K a power of two: exact)
-      int i = m >> lc.k_shift;
-      double f = ((double)(m & ((1 << lc.k_shift) - 1)) + fs) * lc.inv_k;
-      // the clamp's ends: u <= -1 or NaN, and the degenerate grids
-      const bool first = !lc.const_last && !inside && lc.a_pos && u_in >= -1.;
-      const bool to_last = lc.const_last || (!inside && !first);
-      i = first ? 0 : to_last ? lc.last : i;
-      f = first ? 0. : to_last ? 1. : f;
+      dl = fmax(-0.5, fmin(dl, 1.0)); // beyond the sub-cell by more than one: the clamp below decides
+      double p = fma(dl, 0.13147226220077304, -0.16626609150418023);
+      p = fma(p, dl, 0.1999935135656574);
+      p = fma(p, dl, -0.24999995348000387);
+      p = fma(p, dl, 0.3333333332203152);
+      p = fma(p, dl, -0.4999999999999832);
+      const double l = fma(dl * dl, p, dl); // log1p(dl)
+      double idx = ((double)m + fma(lc.s, l, lc.off)) * lc.inv_k;
+      idx = fmax(0., fmin(idx, lc.top));
+      const int i = min((int)idx, lc.last);
+      const double f = idx - (double)i;
       const NT *d = device_data_ptr + i;
       return dfrg::gld(d) * (1. - f) + dfrg::gld(d + 1) * f;
     }
