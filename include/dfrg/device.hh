@@ -130,23 +130,6 @@ namespace dfrg
       return y;
     }
 
-    // Block sum in a fixed order: wave sums to LDS, then wave 0 adds them in index order.
-    // `smem` needs blockDim.x / 64 doubles.  Returns the total to every thread of the block.
-    __device__ __forceinline__ double block_sum(double v, double *smem)
-    {
-      const int lane = threadIdx.x & (wave - 1);
-      const int wid = threadIdx.x / wave;
-      const int nw = (blockDim.x + wave - 1) / wave;
-      v = wave_sum(v);
-      __syncthreads();
-      if (lane == 0) smem[wid] = v;
-      __syncthreads();
-      double t = 0.0;
-      for (int i = 0; i < nw; ++i) t += smem[i];
-      __syncthreads();
-      return t;
-    }
-
     // ------------------------------------------------------------------------------------------
     // Cross-block publication without cache-wide fences.  Each XCD has its own L2, so a release
     // fence at device scope writes back the whole L2 and an acquire fence invalidates it, which
@@ -231,7 +214,7 @@ namespace dfrg
         for (int c = 0; c < n_slots; c += 64) {
           const int j = c + (int)threadIdx.x;
           const double v = j < n_slots ? fetch(&partials[(long long)(first_slot + j) * kSlotStride]) : 0.0;
-          t += wave_sum(v);
+          t += wave_sum1(v);
         }
         if (threadIdx.x == 0) {
           *total = t;
