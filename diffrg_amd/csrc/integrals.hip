@@ -351,8 +351,8 @@ namespace
   // table-driven log and exp (device.hh), take 50 to the same accuracy (against long double, over
   // 1,300 integrals of all orders and table sizes: largest error 6.1e-16, 6.0e-16 before).  The cell
   // is floor of the FP64 index as in the reference, so the interpolation's kinks stay where they
-  // are.  1,023 uneven integrals (87M evaluations): 502 -> 151 us; 64 integrals of {64, 32, 32}
-  // nodes: 31.9 -> 12.0 us.  For integrals with a coordinate map of bias >= 2 whose log argument stays
+  // are.  1,023 uneven integrals (87M evaluations): 502 -> 149 us; 64 integrals of {64, 32, 32}
+  // nodes: 31.9 -> 11.7 us.  For integrals with a coordinate map of bias >= 2 whose log argument stays
   // positive, finite table values and |64 t| < 2^30 (rule in dfrg_se_batch_create); the others keep
   // se_G_fp64.
   struct SESeeded {
