@@ -175,15 +175,11 @@ namespace
   };
 
   // A frequency pair f(q,w) + f(q,-w) = RBdot (d2p + d2m)/(d1^2 d2p d2m) takes one reciprocal of the
-  // product of its denominators (16 VALU against 45 for three IEEE divisions; FP64 mode rcp_f64,
-  // mixed mode the FP32-seeded rcp_seeded).  The denominators are formed times `scale`, so their product
-  // stays in range at any k; scale is a power of two and changes no rounding.
-  template <int MODE> __device__ __forceinline__ double ft_rcp(double d)
-  {
-    return MODE == DFRG_FP64 ? dev::rcp_f64(d) : dev::rcp_seeded(d);
-  }
-
-  template <int MODE, int BLOCK> __global__ __launch_bounds__(BLOCK) void ft_kernel(FTArgs A)
+  // product of its denominators (16 VALU against 45 for three IEEE divisions), in both modes by rcp_f64.  An FP32
+  // seed in mixed mode, at 24.0 us against 25.8 for 8,191 integrals of 48 nodes, lost terms without a sign
+  // where k is below 1e-5 of a mass: a product of three denominators leaves the FP32 range.  The denominators
+  // are formed times `scale`, a power of two, which changes no rounding.
+  template <int BLOCK> __global__ __launch_bounds__(BLOCK) void ft_kernel(FTArgs A)
   {
     extern __shared__ double sm[];
     const int nx = A.nx;
@@ -227,7 +223,7 @@ namespace
       s_a1[j] = a1;
       s_a2[j] = a2;
       if (T > 0) {
-        const double d2 = p0 * p0 + a2, r = ft_rcp<MODE>(a1 * d2);
+        const double d2 = p0 * p0 + a2, r = dev::rcp_f64(a1 * d2);
         acc += f * (T * (r * (r * d2)));
       }
     }
@@ -248,7 +244,7 @@ namespace
         const double d1 = w2 + s_a1[j];
         const double d2p = dp2 + a2, d2m = dm2 + a2;
         const double D2 = d2p * d2m;
-        const double r = ft_rcp<MODE>(d1 * D2);
+        const double r = dev::rcp_f64(d1 * D2);
         s = fma(s_f[j], (d2p + d2m) * (r * (r * D2)), s);
       };
       if (lp == 6) { // one radial node per wave: a uniform loop (28.0 -> 25.8 us below)
@@ -1012,20 +1008,11 @@ int dfrg_ft_batch(int d, int radial_mode, int n_int, const double *d_T, const do
   }
   hipStream_t s = resolve_stream(stream);
   const size_t shm = sizeof(double) * (3 * nx + B / 64);
-  if (mode == DFRG_FP64) {
-    switch (B) {
-    case 64: hipLaunchKernelGGL((ft_kernel<DFRG_FP64, 64>), dim3(n_int), dim3(64), shm, s, a); break;
-    case 128: hipLaunchKernelGGL((ft_kernel<DFRG_FP64, 128>), dim3(n_int), dim3(128), shm, s, a); break;
-    case 256: hipLaunchKernelGGL((ft_kernel<DFRG_FP64, 256>), dim3(n_int), dim3(256), shm, s, a); break;
-    default: hipLaunchKernelGGL((ft_kernel<DFRG_FP64, 512>), dim3(n_int), dim3(512), shm, s, a); break;
-    }
-  } else {
-    switch (B) {
-    case 64: hipLaunchKernelGGL((ft_kernel<DFRG_MIXED, 64>), dim3(n_int), dim3(64), shm, s, a); break;
-    case 128: hipLaunchKernelGGL((ft_kernel<DFRG_MIXED, 128>), dim3(n_int), dim3(128), shm, s, a); break;
-    case 256: hipLaunchKernelGGL((ft_kernel<DFRG_MIXED, 256>), dim3(n_int), dim3(256), shm, s, a); break;
-    default: hipLaunchKernelGGL((ft_kernel<DFRG_MIXED, 512>), dim3(n_int), dim3(512), shm, s, a); break;
-    }
+  switch (B) {
+  case 64: hipLaunchKernelGGL(ft_kernel<64>, dim3(n_int), dim3(64), shm, s, a); break;
+  case 128: hipLaunchKernelGGL(ft_kernel<128>, dim3(n_int), dim3(128), shm, s, a); break;
+  case 256: hipLaunchKernelGGL(ft_kernel<256>, dim3(n_int), dim3(256), shm, s, a); break;
+  default: hipLaunchKernelGGL(ft_kernel<512>, dim3(n_int), dim3(512), shm, s, a); break;
   }
   DFRG_LAUNCHED("ft_kernel");
   return DFRG_OK;

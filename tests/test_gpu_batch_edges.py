@@ -82,3 +82,50 @@ def test_finite_T_sizes(gpu, qp, nm, nx, k, radial_mode):
                 assert np.abs(out.to_host() / ref - 1).max() <= TOL
     finally:
         gpu.ft_set_block(0)
+
+
+def _ft(gpu, T, p0, pabs, m1, m2, rules, x, w, extent, k, d, radial_mode, block, tol=TOL):
+    """ft_batch in both modes against the oracle: finite values to `tol`, zeros, infinities and NaNs alike."""
+    T, p0, pabs, m1, m2 = np.broadcast_arrays(*(np.asarray(a, float) for a in (T, p0, pabs, m1, m2)))
+    # the oracle adds the zero mode beside its first node: a node of weight 0 where there is none
+    with np.errstate(all="ignore"):
+        ref = O.c2_finiteT(T, p0, pabs, m1, m2, [r if len(r[0]) else (np.ones(1), np.zeros(1)) for r in rules],
+                           x, w, extent, k, 1.0, d, radial_mode)
+    lens = np.array([len(r[0]) for r in rules], np.int32)
+    off = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32)
+    pad = np.ones(1)  # the concatenation may be empty
+    A = gpu.DeviceArray.from_host
+    dev = {"T": A(T), "p0": A(p0), "pabs": A(pabs), "m1": A(m1), "m2": A(m2),
+           "mx": A(np.concatenate([r[0] for r in rules] + [pad])),
+           "mw": A(np.concatenate([r[1] for r in rules] + [pad])),
+           "m_off": A(off), "m_n": A(lens), "x": A(x), "w": A(w)}
+    out = gpu.DeviceArray(len(T))
+    try:
+        gpu.ft_set_block(block)
+        for mode in (gpu.FP64, gpu.MIXED):
+            print(f"[case] finite-T k={k} nx={len(x)} radial_mode={radial_mode} block={block} mode={mode}", flush=True)
+            gpu.ft_batch(dev, out, extent, k, mode, d, radial_mode)
+            got = out.to_host()
+            fin = np.isfinite(ref) & (ref != 0)
+            assert np.array_equal(got[~fin], ref[~fin], equal_nan=True), (got, ref)
+            assert np.all(np.abs(got[fin] / ref[fin] - 1) <= tol), np.abs(got / ref - 1)
+    finally:
+        gpu.ft_set_block(0)
+
+
+# the direction every flow runs: k falls while temperature, momenta and masses stay (products of three
+# denominators over k^2 leave the FP32 range near k = 1e-6); and masses that stay where k grows
+@pytest.mark.parametrize("k", [1e-3, 1e-5, 3e-6, 1e-6, 1e-8, 1e-15, 1e6])
+@pytest.mark.parametrize("radial_mode", [0, 1])
+@pytest.mark.parametrize("block", [0, 64])
+def test_finite_T_scale_against_fixed_masses(gpu, qp, k, radial_mode, block):
+    rng = np.random.default_rng(5)
+    n = 8
+    T = np.array([0.05, 0.1, 0.3, 0.0, 0.1, 2.0, 0.1, 0.3])
+    rules = [(2 * np.pi * max(t, 0.1) * np.arange(1, m + 1), np.full(m, max(t, 0.1)))
+             for t, m in zip(T, (64, 96, 17, 48, 3, 66, 130, 33))]
+    m1, m2 = rng.uniform(0.01, 3, n), rng.uniform(0.01, 3, n)
+    m1[4], m2[4] = 1e4, 1e-4
+    extent = 6.0 * k if radial_mode else 20.0
+    _ft(gpu, T, 2 * np.pi * T * rng.integers(0, 5, n), rng.uniform(0, 1, n), m1, m2, rules, qp.get_points(48),
+        qp.get_weights(48), extent, k, 4, radial_mode, block)
