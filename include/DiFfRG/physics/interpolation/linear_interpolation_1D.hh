@@ -18,13 +18,15 @@
 // FP64 rounding (~1e-14 of a cell); the clamp to [0, N-1] and the reference's NaN rule (fmax(0, fmin(NaN,
 // N-1)): a NaN index takes the last point) give the ends: u <= -1 takes the first point when u = -1 and
 // a > 0 (index -inf), the last point otherwise (NaN, or +inf for a < 0); N = 1, bias 0 and NaN bias
-// have a NaN or zero-width index: the last point.  The device code has no branch on the grid, so a
+// have a NaN or zero-width index: the last point.  On the device u below -1 or NaN counts as -1, where
+// the sum is past the first end for a > 0 and past the last for a < 0 whatever the bias, and an o of 1e300
+// moves it past the last end where u is not -1 itself.  The device code has no branch on the grid, so a
 // user KERNEL's loop-invariant lookups (at q alone) stay hoistable.  Biases beyond +-700 (exp
 // overflows) and grids of more than 2^21 sub-cells per unit of log2 are refused.
 //
 // VALU issue bounds a KERNEL made of lookups, exponentials and divisions: with sub-cells of 1/4, an
 // atanh series to z^17 and the sub-cell corrected by selects, 64 requests of {64, 32, 32} nodes took
-// 33.9 us in the kernel, now 29.7 (155 -> 129 VALU instructions per node).
+// 33.9 us in the kernel, now 29.7 (155 -> 127 VALU instructions per node).
 #pragma once
 
 #include <cmath>
@@ -123,7 +125,6 @@ namespace DiFfRG
       double s = 0, s_ln2 = 0;       // K(N-1)/a, K(N-1)/a ln 2
       double off = 0;                // o
       double inv_k = 1;              // 1/K
-      double u_first = 0, u_last = 0; // stand-ins for u = -1 (a > 0: the first point) and for u < -1 or NaN
       double top = 0;                // N - 1
       int m_last = 0;                // last sub-cell (K(N-1) - 1)
       int last = 0;                  // last cell (N - 2; 0 for N = 1)
@@ -159,17 +160,12 @@ namespace DiFfRG
         L.off = a > 0 ? 0. : 1.;
         L.inv_k = 1. / K;
         L.m_last = int(subs) - 1;
-        L.u_last = a > 0 ? 1e300 : -1. + 0x1p-53;
-        L.u_first = a > 0 ? 0. : L.u_last;
       } else {
         // one point, bias 0 or NaN: the reference's index is 0 x (...)/a with a NaN or infinite
         // factor, or the one point; all points take the last point.  A valid dummy table keeps the
         // device code branch-free.
         h = {make_double2(0., 1.)};
         L.inv_b = std::numeric_limits<double>::quiet_NaN();
-        L.u_first = L.u_last = 1e300;
-        L.s = 2.;
-        L.inv_k = 1e12;
       }
       void *p = nullptr;
       dfrg::check(dfrg_malloc(&p, sizeof(double2) * h.size()), "LinearInterpolator1D cells");
@@ -183,10 +179,9 @@ namespace DiFfRG
     // the lerp at the reference's index of u = (x - c)/b (device, no branch on the grid)
     __device__ __forceinline__ NT log_cell_lerp(const double u_in) const
     {
-      // u > -1 (false for NaN), or a stand-in beyond the grid's end
-      const double u_first = lc.u_first, u_last = lc.u_last;
-      const double beyond = u_in == -1. ? u_first : u_last;
-      const double u = u_in > -1. ? u_in : beyond;
+      const double o = lc.off;
+      const double off = u_in >= -1. ? o : 1e300; // 1e300: past the last point
+      const double u = fmax(u_in, -1.);           // -1 for NaN
       // sub-cell estimate: log2(1 + u) = e + log2(mant), mant in [1/2, 1), FP32 log of the mantissa
       const double w = 1. + u;
       const double lg = (double)__builtin_amdgcn_logf((float)__builtin_amdgcn_frexp_mant(w));
@@ -201,7 +196,7 @@ namespace DiFfRG
       p = fma(p, dl, 0.3333333332203152);
       p = fma(p, dl, -0.4999999999999832);
       const double l = fma(dl * dl, p, dl); // log1p(dl)
-      double idx = ((double)m + fma(lc.s, l, lc.off)) * lc.inv_k;
+      double idx = ((double)m + fma(lc.s, l, off)) * lc.inv_k;
       idx = fmax(0., fmin(idx, lc.top));
       const int i = min((int)idx, lc.last);
       const double f = idx - (double)i;

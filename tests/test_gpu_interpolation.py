@@ -274,6 +274,26 @@ def test_fp64_log_coordinates_on_the_device(kat, n, bias, start, stop):
     assert np.max(np.abs(dev - host)) <= slope * tol_idx + 4 * 2.0 ** -52
 
 
+@pytest.mark.parametrize("bias", [-3.0, -36.0, -37.0, -50.0, -100.0, -700.0, 36.0, 650.0, 691.0, 700.0])
+@pytest.mark.parametrize("n,stop", [(64, 1.0), (3, 8.0), (500, 0.25)])
+def test_fp64_log_coordinates_ends_at_large_bias(kat, bias, n, stop):
+    """Beyond the grid's ends the index is the first or last point exactly, whatever the bias: for a negative one
+    x = stop already has u = -1 (expm1(bias) rounds to -1 below about -37), where every larger x and NaN
+    follow; for a positive one u < -1 and NaN take the last point, u = -1 the first.  The intervals are powers of
+    two, so the device's product with 1/b and the reference's division by b agree."""
+    with np.errstate(all="ignore"):
+        b = stop / np.expm1(np.float64(bias))
+    pts = np.array([1.5 * stop, 2.0 * stop, 1e300, np.inf, np.nan, -np.inf, -1e300])
+    if bias < 0:
+        pts = np.concatenate([pts, [stop] if bias < -40 else [], [-0.5 * stop, -stop]])
+    else:
+        pts = np.concatenate([pts, [-2.0 * b, -1.5 * b, -stop]])
+    lin = np.arange(n, dtype=np.float64) * 0.75 - 3.0
+    want = lin[log_index64(pts, n, 0.0, stop, bias).astype(int)]
+    dev, host = run(kat, 8, [n, 0.0, stop, bias], lin, pts)
+    assert np.all(np.isin(want, lin[[0, -1]])) and np.array_equal(dev, want), (dev, want)
+
+
 def test_fp64_log_coordinates_refused_bias(kat):
     # beyond |bias| = 700 exp(bias) overflows; the device index refuses such grids at construction
     cp = np.array([16, 0.0, 1.0, 800.0])
