@@ -174,6 +174,14 @@ namespace
     double *out;
   };
 
+  // Lanes, as a power of two, that a chunk of `rest` Matsubara nodes takes: 64, or for a last chunk of at
+  // most 32 the next power of two (at least 2), with 64 >> it radial nodes at once, so short rules and
+  // remainders do not leave lanes idle.
+  constexpr int ft_log2_lanes(int rest) { return rest > 32 ? 6 : rest > 2 ? 32 - __builtin_clz(rest - 1) : 1; }
+  static_assert(ft_log2_lanes(0) == 1 && ft_log2_lanes(2) == 1 && ft_log2_lanes(3) == 2 && ft_log2_lanes(4) == 2 &&
+                ft_log2_lanes(5) == 3 && ft_log2_lanes(16) == 4 && ft_log2_lanes(17) == 5 && ft_log2_lanes(32) == 5 &&
+                ft_log2_lanes(33) == 6);
+
   // A frequency pair f(q,w) + f(q,-w) = RBdot (d2p + d2m)/(d1^2 d2p d2m) takes one reciprocal of the
   // product of its denominators (16 VALU against 45 for three IEEE divisions), in both modes by rcp_f64.  An FP32
   // seed in mixed mode, at 24.0 us against 25.8 for 8,191 integrals of 48 nodes, lost terms without a sign
@@ -192,13 +200,9 @@ namespace
     const double T = A.T[i], pa = A.pabs[i], m1 = A.m1[i], m2 = A.m2[i], p0 = A.p0[i] * A.root;
     const int off = A.m_off[i], nm = A.m_n[i];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    // lanes (as a power of two) a chunk of `rest` Matsubara nodes takes: 64, or for a last chunk of at
-    // most 32 the next power of two, with 64 >> it radial nodes at once, so short rules and remainders
-    // do not leave lanes idle
-    auto log2_lanes = [](int rest) { return rest > 32 ? 6 : 32 - __builtin_clz((rest - 1) | 1); };
     // this lane's first Matsubara node, loaded before the q-only terms so the two loads overlap
     double wn0 = 0.0, wgt0 = 0.0;
-    const int nl0 = lane & ((1 << log2_lanes(nm)) - 1);
+    const int nl0 = lane & ((1 << ft_log2_lanes(nm)) - 1);
     if (nl0 < nm) {
       wn0 = A.mx[off + nl0];
       wgt0 = A.mw[off + nl0];
@@ -232,7 +236,7 @@ namespace
     // are LDS reads shared by the lanes
     constexpr int NW = BLOCK / 64;
     for (int n0 = 0; n0 < nm; n0 += 64) {
-      const int rest = nm - n0, lp = log2_lanes(rest);
+      const int rest = nm - n0, lp = ft_log2_lanes(rest);
       const int n = n0 + (lane & ((1 << lp) - 1));
       if (n >= nm) break;
       const double wn = A.root * (n0 == 0 ? wn0 : A.mx[off + n]), wgt = n0 == 0 ? wgt0 : A.mw[off + n];

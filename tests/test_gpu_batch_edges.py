@@ -129,3 +129,13 @@ def test_finite_T_scale_against_fixed_masses(gpu, qp, k, radial_mode, block):
     extent = 6.0 * k if radial_mode else 20.0
     _ft(gpu, T, 2 * np.pi * T * rng.integers(0, 5, n), rng.uniform(0, 1, n), m1, m2, rules, qp.get_points(48),
         qp.get_weights(48), extent, k, 4, radial_mode, block)
+
+
+@pytest.mark.parametrize("block", [0, 64])
+@pytest.mark.parametrize("nx", [1, 48])
+def test_finite_T_zero_mode_alone(gpu, qp, nx, block):
+    # integrals without Matsubara nodes: the zero mode, or nothing at T = 0.  (The lanes' share of such a rule
+    # is a static_assert beside the kernel.)
+    T = np.array([0.1, 0.0, 0.3])
+    rules = [(np.zeros(0), np.zeros(0))] * 2 + [(np.array([1.0]), np.array([0.3]))]
+    _ft(gpu, T, 0.3, 0.7, 0.5, 0.25, rules, qp.get_points(nx), qp.get_weights(nx), 20.0, 1.0, 4, 0, block)
