@@ -170,7 +170,7 @@ namespace
     const int *m_off, *m_n;
     const double *x, *w;
     double extent, k, pref;
-    double scale, root; // a power of four near 1/k^2, and its root
+    double limit; // largest square of a momentum, frequency or mass in the fast form (0: never)
     double *out;
   };
 
@@ -182,24 +182,33 @@ namespace
                 ft_log2_lanes(5) == 3 && ft_log2_lanes(16) == 4 && ft_log2_lanes(17) == 5 && ft_log2_lanes(32) == 5 &&
                 ft_log2_lanes(33) == 6);
 
-  // A frequency pair f(q,w) + f(q,-w) = RBdot (d2p + d2m)/(d1^2 d2p d2m) takes one reciprocal of the
-  // product of its denominators (16 VALU against 45 for three IEEE divisions), in both modes by rcp_f64.  An FP32
-  // seed in mixed mode, at 24.0 us against 25.8 for 8,191 integrals of 48 nodes, lost terms without a sign
-  // where k is below 1e-5 of a mass: a product of three denominators leaves the FP32 range.  The denominators
-  // are formed times `scale`, a power of two, which changes no rounding.
+  // Both modes evaluate the same FP64 arithmetic, in one of two forms per integral.
+  // Fast: a frequency pair f(q,w) + f(q,-w) = RBdot (d2p + d2m)/(d1^2 d2p d2m) takes one reciprocal of the
+  // product of its denominators (15 VALU against 45 for three IEEE divisions).  The product has to stay in
+  // range: with k in [2^-80, 2^80] and q^2 + |p|^2 + |m1| + |m2| + p0^2 and w^2 below 2^246 (kFtLimit), every
+  // denominator is below 2^249, so 1/(d1^2 d2p d2m) is above 2^-996, and a denominator that cancels (two
+  // subtractions) is zero or above 2^-106 k^2, so the product of three does not underflow.
+  // General: three IEEE divisions per pair, as in the reference.  For integrals beyond those limits, whose
+  // accumulator becomes NaN, and for those whose fast sum is not finite (a vanishing denominator makes
+  // the reciprocal NaN): a sum that is not finite sends its block through this form.
+  // (An FP32 seed in mixed mode, at 24.0 us against 25.8 for 8,191 integrals of 48 nodes, lost terms without a
+  // sign where k is below 1e-5 of a mass: the product of three denominators leaves the FP32 range.)
+  constexpr double kFtLimit = 0x1p246;
   template <int BLOCK> __global__ __launch_bounds__(BLOCK) void ft_kernel(FTArgs A)
   {
     extern __shared__ double sm[];
     const int nx = A.nx;
-    double *s_f = sm;            // element * weight * RBdot * scale^3
-    double *s_a1 = sm + nx;      // (q^2 + R(q^2) + m1) scale
-    double *s_a2 = sm + 2 * nx;  // (q^2 + |p|^2 + R(q^2 + |p|^2) + m2) scale
-    double *s_red = sm + 3 * nx; // block reduction
+    double *s_f = sm;            // element * weight * RBdot (general form: element * weight)
+    double *s_a1 = sm + nx;      // q^2 + R(q^2) + m1
+    double *s_a2 = sm + 2 * nx;  // q^2 + |p|^2 + R(q^2 + |p|^2) + m2
+    double *s_rd = sm + 3 * nx;  // general form: RBdot
+    double *s_red = sm + 4 * nx; // block reduction
     const int i = blockIdx.x;
-    const double k = A.k, k2 = k * k, sc = A.scale;
-    const double T = A.T[i], pa = A.pabs[i], m1 = A.m1[i], m2 = A.m2[i], p0 = A.p0[i] * A.root;
+    const double k = A.k, k2 = k * k;
+    const double T = A.T[i], pa = A.pabs[i], m1 = A.m1[i], m2 = A.m2[i], p0 = A.p0[i];
     const int off = A.m_off[i], nm = A.m_n[i];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    constexpr int NW = BLOCK / 64;
     // this lane's first Matsubara node, loaded before the q-only terms so the two loads overlap
     double wn0 = 0.0, wgt0 = 0.0;
     const int nl0 = lane & ((1 << ft_log2_lanes(nm)) - 1);
@@ -207,9 +216,11 @@ namespace
       wn0 = A.mx[off + nl0];
       wgt0 = A.mw[off + nl0];
     }
-    double acc = 0.0;
-    // q-only terms, and the zero mode T f(q, 0) of sum = T f(0) + sum_n w_n (f(x_n) + f(-x_n))
-    for (int j = threadIdx.x; j < nx; j += BLOCK) {
+    // the q-only terms of radial node j; `qp2` = q^2 + |p|^2
+    struct QTerms {
+      double elw, rdot, a1, a2, qp2;
+    };
+    auto q_terms = [&](int j) {
       double q, el;
       if (A.radial_mode == 0) {
         q = k * sqrt(A.x[j] * A.extent);
@@ -218,37 +229,55 @@ namespace
         q = A.extent * A.x[j];
         el = A.pref * ipow_dev(q, A.d - 2);
       }
-      const double q2 = q * q, xr = q2 / k2, e = exp(-xr);
-      const double f = el * (A.w[j] * A.extent) * (2.0 * e * k2 * (1.0 + xr)) * sc * sc * sc;
-      const double qp2 = q2 + pa * pa;
-      const double a1 = (q2 + k2 * e + m1) * sc;
-      const double a2 = (qp2 + k2 * exp(-(qp2 / k2)) + m2) * sc;
+      const double q2 = q * q, xr = q2 / k2, e = exp(-xr), qp2 = q2 + pa * pa;
+      return QTerms{el * (A.w[j] * A.extent), 2.0 * e * k2 * (1.0 + xr), q2 + k2 * e + m1,
+                    qp2 + k2 * exp(-(qp2 / k2)) + m2, qp2};
+    };
+    // the block's sum, in every lane
+    auto block_total = [&](double v) {
+      double t = dev::wave_sum1(v);
+      if (NW > 1) {
+        if (lane == 0) s_red[wv] = t;
+        __syncthreads();
+        t = s_red[0];
+        for (int u = 1; u < NW; ++u) t += s_red[u];
+      }
+      return t;
+    };
+    const double ext2 = fabs(m1) + fabs(m2) + p0 * p0;
+    const bool fast = ext2 + pa * pa < A.limit; // block-uniform
+    double acc = fast ? 0.0 : NAN;
+    // q-only terms, and the zero mode T f(q, 0) of sum = T f(0) + sum_n w_n (f(x_n) + f(-x_n))
+    for (int j = threadIdx.x; j < nx; j += BLOCK) {
+      const QTerms t = q_terms(j);
+      const double f = t.elw * t.rdot;
       s_f[j] = f;
-      s_a1[j] = a1;
-      s_a2[j] = a2;
+      s_a1[j] = t.a1;
+      s_a2[j] = t.a2;
       if (T > 0) {
-        const double d2 = p0 * p0 + a2, r = dev::rcp_f64(a1 * d2);
+        const double d2 = p0 * p0 + t.a2, r = dev::rcp_normal(t.a1 * d2);
         acc += f * (T * (r * (r * d2)));
       }
+      if (!(t.qp2 + ext2 < A.limit)) acc = NAN;
     }
     __syncthreads();
     // Matsubara nodes across the lanes (fixed per lane), radial nodes across the waves; the q terms
     // are LDS reads shared by the lanes
-    constexpr int NW = BLOCK / 64;
-    for (int n0 = 0; n0 < nm; n0 += 64) {
+    for (int n0 = 0; n0 < nm && fast; n0 += 64) {
       const int rest = nm - n0, lp = ft_log2_lanes(rest);
       const int n = n0 + (lane & ((1 << lp) - 1));
       if (n >= nm) break;
-      const double wn = A.root * (n0 == 0 ? wn0 : A.mx[off + n]), wgt = n0 == 0 ? wgt0 : A.mw[off + n];
+      const double wn = n0 == 0 ? wn0 : A.mx[off + n], wgt = n0 == 0 ? wgt0 : A.mw[off + n];
       const double dp = wn + p0, dm = -wn + p0;
       const double w2 = wn * wn, dp2 = dp * dp, dm2 = dm * dm;
+      if (!(w2 < kFtLimit)) acc = NAN;
       double s = 0.0;
       auto term = [&](int j) {
         const double a2 = s_a2[j];
         const double d1 = w2 + s_a1[j];
         const double d2p = dp2 + a2, d2m = dm2 + a2;
         const double D2 = d2p * d2m;
-        const double r = dev::rcp_f64(d1 * D2);
+        const double r = dev::rcp_normal(d1 * D2);
         s = fma(s_f[j], (d2p + d2m) * (r * (r * D2)), s);
       };
       if (lp == 6) { // one radial node per wave: a uniform loop (28.0 -> 25.8 us below)
@@ -261,11 +290,32 @@ namespace
       }
       acc = fma(wgt, s, acc);
     }
-    double tot = dev::wave_sum1(acc);
-    if (NW > 1) {
-      if (lane == 0) s_red[wv] = tot;
+    double tot = block_total(acc);
+    if (!isfinite(tot)) { // block-uniform: the general form
+      __syncthreads();    // every wave has read the fast form's terms and s_red
+      acc = 0.0;
+      for (int j = threadIdx.x; j < nx; j += BLOCK) {
+        const QTerms t = q_terms(j);
+        s_f[j] = t.elw;
+        s_rd[j] = t.rdot;
+        s_a1[j] = t.a1;
+        s_a2[j] = t.a2;
+        if (T > 0) {
+          const double g1 = 1.0 / t.a1, g2 = 1.0 / (p0 * p0 + t.a2);
+          acc += t.elw * (T * (t.rdot * g1 * g1 * g2));
+        }
+      }
       __syncthreads();
-      for (int u = 1; wv == 0 && u < NW; ++u) tot += s_red[u];
+      for (int n = lane; n < nm; n += 64) {
+        const double wn = A.mx[off + n], wgt = A.mw[off + n], dp = wn + p0, dm = -wn + p0;
+#pragma unroll 2
+        for (int j = wv; j < nx; j += NW) {
+          const double rd = s_rd[j], a2 = s_a2[j];
+          const double g1 = 1.0 / (wn * wn + s_a1[j]), gp = 1.0 / (dp * dp + a2), gm = 1.0 / (dm * dm + a2);
+          acc += s_f[j] * (wgt * (rd * g1 * g1 * gp + rd * g1 * g1 * gm));
+        }
+      }
+      tot = block_total(acc);
     }
     if (threadIdx.x == 0) A.out[i] = tot;
   }
@@ -995,12 +1045,9 @@ int dfrg_ft_batch(int d, int radial_mode, int n_int, const double *d_T, const do
   DFRG_CHECK_ARG(d_T && d_p0 && d_pabs && d_m1 && d_m2 && d_mx && d_mw && d_m_off && d_m_n && d_x && d_w && d_out,
                  "NULL device pointer");
   FTArgs a{d, radial_mode, n_int, nx, d_T, d_p0, d_pabs, d_m1, d_m2, d_mx, d_mw, d_m_off, d_m_n, d_x, d_w,
-           extent, k, 0.0, 1.0, 1.0, d_out};
+           extent, k, 0.0, 0.0, d_out};
   a.pref = S_d_host(d - 1) / std::pow(2.0 * kPi, d - 1);
-  if (std::isnormal(k)) {
-    a.root = std::ldexp(1.0, -std::ilogb(k));
-    a.scale = a.root * a.root;
-  }
+  if (std::fabs(k) >= 0x1p-80 && std::fabs(k) <= 0x1p80) a.limit = kFtLimit;
   // threads per integral: the caller's choice (dfrg_ft_set_block), else enough waves for about
   // two per SIMD over the whole batch, 1 to 8 per integral and not more than radial nodes
   int B = g_ft_block;
@@ -1011,7 +1058,7 @@ int dfrg_ft_batch(int d, int radial_mode, int n_int, const double *d_T, const do
     B = 64 * nw;
   }
   hipStream_t s = resolve_stream(stream);
-  const size_t shm = sizeof(double) * (3 * nx + B / 64);
+  const size_t shm = sizeof(double) * (4 * nx + B / 64);
   switch (B) {
   case 64: hipLaunchKernelGGL(ft_kernel<64>, dim3(n_int), dim3(64), shm, s, a); break;
   case 128: hipLaunchKernelGGL(ft_kernel<128>, dim3(n_int), dim3(128), shm, s, a); break;

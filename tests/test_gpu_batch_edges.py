@@ -131,6 +131,45 @@ def test_finite_T_scale_against_fixed_masses(gpu, qp, k, radial_mode, block):
         qp.get_weights(48), extent, k, 4, radial_mode, block)
 
 
+@pytest.mark.parametrize("block", [0, 64, 512])
+@pytest.mark.parametrize("k", [1.0, 1e-40, 1e40])
+def test_finite_T_huge_masses(gpu, qp, k, block):
+    # masses past the range of a product of denominators, infinite and NaN ones: 0, the small value or NaN, and
+    # ordinary neighbours beside them; scales k where such products leave the FP64 range altogether
+    k2 = k * k
+    m1 = np.array([0.5, 1.0, 1.0, 1.0, 1.0, 1e60, np.inf, np.nan, 1.0, 1e60, -0.5]) * k2
+    m2 = np.array([0.5, 1e120 / k2, 1e160 / k2, np.inf, np.nan, 1.0, 1.0, 1.0, -np.inf, 1e110, 0.25]) * k2
+    n = len(m1)
+    T = np.where(np.arange(n) % 2, 0.1, 0.0) * k
+    rules = [(2 * np.pi * 0.1 * k * np.arange(1, m + 1), np.full(m, 0.1 * k))
+             for m in (64, 65, 5, 130, 1, 33, 64, 2, 17, 64, 66)]
+    _ft(gpu, T, 0.3 * k, 0.7 * k, m1, m2, rules, qp.get_points(37), qp.get_weights(37), 20.0, k, 4, 0, block)
+
+
+@pytest.mark.parametrize("block", [0, 256])
+def test_finite_T_huge_external_and_frequencies(gpu, qp, block):
+    p0 = np.array([0.3, 1e80, 1e120, np.inf, 0.3, 0.3, 0.3])
+    pabs = np.array([0.7, 0.7, 0.7, 0.7, 1e90, np.inf, 0.7])
+    rules = [(np.geomspace(1e-3, top, m), np.full(m, 0.1)) for top, m in
+             ((10.0, 64), (10.0, 65), (10.0, 64), (10.0, 33), (10.0, 5), (10.0, 64), (1e95, 130))]
+    _ft(gpu, 0.1, p0, pabs, 0.5, 0.25, rules, qp.get_points(37), qp.get_weights(37), 20.0, 1.0, 4, 0, block)
+
+
+@pytest.mark.parametrize("block", [0, 64])
+def test_finite_T_vanishing_denominators(gpu, qp, block):
+    # one radial node at q^2 = 49, whose regulator e^-49 is below a rounding, so the masses cancel q^2 exactly:
+    # a zero d1 in the zero mode, a zero d2 there and in a frequency pair: infinite, as by three divisions
+    x, w = np.array([0.98]), np.array([1.0])
+    q2 = float(np.sqrt(0.98 * 50.0) ** 2)
+    assert q2 + np.exp(-q2) == q2
+    rules = [(np.array([0.5, 2.0]), np.array([0.1, 0.1]))] * 5
+    T = np.array([0.1, 0.1, 0.0, 0.0, 0.1])
+    p0 = np.array([0.3, 0.0, 2.0, 0.3, 0.3])
+    m1 = np.array([-q2, 0.5, 0.5, -q2, 0.5])
+    m2 = np.array([0.25, -q2, -q2, 0.25, 0.25])
+    _ft(gpu, T, p0, 0.0, m1, m2, rules, x, w, 50.0, 1.0, 4, 0, block)
+
+
 @pytest.mark.parametrize("block", [0, 64])
 @pytest.mark.parametrize("nx", [1, 48])
 def test_finite_T_zero_mode_alone(gpu, qp, nx, block):
