@@ -41,15 +41,21 @@ namespace dfrg
     // tabulated in LDS, an FP64 step is one dependent FMA, and the compensated step has four
     // dependent operations with its error terms beside them; the earlier form took every Newton step
     // in double-double with a three-division quotient per degree.  Order 128: 293 -> 16.8 us, 32: 86 ->
-    // 6.6, 1024: 1972 -> 96.5.
+    // 6.6, 1024: 1972 -> 96.5.  LONG, for orders past kGlTable (half a long vacuum rule): the reciprocals of the
+    // further degrees are formed in the step (one kernel for both: 2% slower up to kGlTable).
     constexpr int kGlBlock = 64;
-    __global__ __launch_bounds__(kGlBlock) void gl_kernel(int n, double *x, double *w)
+    constexpr int kGlTable = 4096; // 64 KB of LDS
+    // 1/j = x + y
+    __device__ __forceinline__ double2 gl_inverse(int j)
     {
-      extern __shared__ double2 s_inv[]; // 1/j = x + y at j - 1, j <= n
-      for (int j = 1 + threadIdx.x; j <= n; j += kGlBlock) {
-        const double hi = 1.0 / j;
-        s_inv[j - 1] = make_double2(hi, fma(-hi, (double)j, 1.0) * hi);
-      }
+      const double hi = 1.0 / j;
+      return make_double2(hi, fma(-hi, (double)j, 1.0) * hi);
+    }
+    template <bool LONG> __global__ __launch_bounds__(kGlBlock) void gl_kernel(int n, double *x, double *w)
+    {
+      extern __shared__ double2 s_inv[]; // 1/j at j - 1, j <= n_tab
+      const int n_tab = LONG ? kGlTable : n;
+      for (int j = 1 + threadIdx.x; j <= n_tab; j += kGlBlock) s_inv[j - 1] = gl_inverse(j);
       __syncthreads();
       const int i = blockIdx.x * kGlBlock + threadIdx.x;
       const bool own = i < (n + 1) / 2;
@@ -61,13 +67,15 @@ namespace dfrg
       // Newton in FP64: P_j = (2 - 1/j) z P_{j-1} - (1 - 1/j) P_{j-2};  P_n' = n (z P_n - P_{n-1})/(z^2 - 1)
       for (int it = 0; it < 8; ++it) {
         double p0 = 1.0, p1 = z;
-#pragma unroll 8
-        for (int j = 2; j <= n; ++j) {
-          const double inv = s_inv[j - 1].x;
+        auto step = [&](double inv) {
           const double p2 = fma((2.0 - inv) * z, p1, -((1.0 - inv) * p0));
           p0 = p1;
           p1 = p2;
-        }
+        };
+#pragma unroll 8
+        for (int j = 2; j <= n_tab; ++j) step(s_inv[j - 1].x);
+        if (LONG)
+          for (int j = kGlTable + 1; j <= n; ++j) step(gl_inverse(j).x);
         const double dz = p1 * fma(z, z, -1.0) / (dn * fma(z, p1, -p0));
         if (n > 1 && own && !middle) z -= dz;
         // the step leaves about dz^2 n^2/6 near the ends, less elsewhere: below an FP64 rounding
@@ -76,9 +84,7 @@ namespace dfrg
       // one pass at the FP64 root with its rounding errors: with u = z P_{j-1} and t = u - P_{j-2},
       // P_j = u + t - t/j; e carries the error of P_j through the same recurrence
       double p0 = 1.0, p1 = z, e0 = 0.0, e1 = 0.0;
-#pragma unroll 4
-      for (int j = 2; j <= n; ++j) {
-        const double2 inv = s_inv[j - 1];
+      auto step = [&](double2 inv) {
         double dt, ds, dp;
         const double u = z * p1, du = fma(z, p1, -u);
         const double t = two_sum(u, -p0, dt);
@@ -92,7 +98,11 @@ namespace dfrg
         p1 = p2;
         e0 = e1;
         e1 = e2;
-      }
+      };
+#pragma unroll 4
+      for (int j = 2; j <= n_tab; ++j) step(s_inv[j - 1]);
+      if (LONG)
+        for (int j = kGlTable + 1; j <= n; ++j) step(gl_inverse(j));
       if (!own) return;
       const double f = n > 1 ? p1 + e1 : 0.0;
       if (n == 1) {
@@ -317,8 +327,13 @@ namespace dfrg
       h[n + i] = wi;
     }
 
-    // LDS of gl_kernel: the reciprocals of 1..order (64 KB at 4096, the largest order)
-    size_t gl_shared(int order) { return sizeof(double2) * order; }
+    void launch_gl(int order, double *x, double *w, hipStream_t s)
+    {
+      const dim3 grid(((order + 1) / 2 + kGlBlock - 1) / kGlBlock);
+      const size_t shm = sizeof(double2) * std::min(order, kGlTable);
+      const auto kernel = order <= kGlTable ? gl_kernel<false> : gl_kernel<true>;
+      hipLaunchKernelGGL(kernel, grid, dim3(kGlBlock), shm, s, order, x, w);
+    }
 
     bool is_close_abs(double a, double b, double eps)
     {
@@ -361,7 +376,7 @@ namespace
       const int h = m / 2;
       double *g = nullptr;
       DFRG_HIP(hipMallocAsync((void **)&g, sizeof(double) * 2 * h, s));
-      hipLaunchKernelGGL(gl_kernel, dim3((h + 1) / 2 / kGlBlock + 1), dim3(kGlBlock), gl_shared(h), s, h, g, g + h);
+      launch_gl(h, g, g + h, s);
       DFRG_LAUNCHED("gl_kernel");
       hipLaunchKernelGGL(matsubara_vacuum_kernel, dim3(h / 64 + 1), dim3(64), 0, s, h, E, g, g + h, d_x, d_w);
       DFRG_LAUNCHED("matsubara_vacuum_kernel");
@@ -388,9 +403,7 @@ int dfrg_gl_generate(int order, double *d_x, double *d_w, void *stream)
   DFRG_TRY(require_init());
   DFRG_CHECK_ARG(order >= 1 && order <= 4096, "Gauss-Legendre order %d out of range [1,4096]", order);
   DFRG_CHECK_ARG(d_x && d_w, "output pointers are NULL");
-  const int roots = (order + 1) / 2;
-  hipLaunchKernelGGL(gl_kernel, dim3((roots + kGlBlock - 1) / kGlBlock), dim3(kGlBlock), gl_shared(order),
-                     resolve_stream(stream), order, d_x, d_w);
+  launch_gl(order, d_x, d_w, resolve_stream(stream));
   DFRG_LAUNCHED("gl_kernel");
   return DFRG_OK;
 }

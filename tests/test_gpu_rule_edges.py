@@ -44,6 +44,26 @@ def test_gl_order_one(gpu):
     assert x[0] == 0.5 and w[0] == 1.0
 
 
+# a vacuum rule's half length at, past and far past the degrees whose reciprocals are tabulated in LDS (the
+# last would need more LDS than a CU has); E = 1/2 maps the lower half onto [0,1] itself
+@pytest.mark.parametrize("h", [4096, 4097, 5001, 11000])
+def test_long_vacuum_rules(gpu, h):
+    print(f"[case] vacuum rule of {2 * h} nodes", flush=True)
+    x, w, T = gpu.matsubara_generate(0.0, 0.5, 2, 32, 128, 2 * h, 0)
+    assert T == 0.0 and len(x) == 2 * h and np.all(np.diff(x) > 0)
+    with mp.workdps(50):
+        for i in (0, h // 3, h // 2, h - 1):
+            mx, mw = _gl_node(h, x[i])
+            assert abs(x[i] - mx) <= 4.5e-16 * mx, (h, i)
+            assert abs(w[i] * 2 * mp.pi - mw) <= 9e-16 * mw, (h, i)  # two more roundings
+            lx = mp.exp(mp.log(5e5) * mx)
+            assert abs(x[h + i] - lx) <= 1e-14 * lx, (h, i)  # 13 roundings of the exponent log(5e5) x, and its own
+            lw = mw * mp.log(5e5) * lx
+            assert abs(w[h + i] * 2 * mp.pi - lw) <= 1.2e-14 * lw, (h, i)
+    qp = gpu.QuadratureProvider(vacuum_quad_size=2 * h)
+    assert np.array_equal(qp.get_matsubara_points(0.0, 0.5), x)
+
+
 # the count's groups of eight steps and their remainders, one and several entries per lane
 @pytest.mark.parametrize("n", [1, 2, 3, 8, 9, 10, 17, 32, 64, 65, 128, 200])
 def test_matsubara_nodes_against_multiprecision(gpu, n):
