@@ -471,9 +471,11 @@ namespace
     return DFRG_OK;
   }
 
-  // Gives the room of the rule placed last back (a rule that could not be made); returns rc.
-  int unplace_rule(dfrg_qp *qp, const Rule &r, int rc)
+  // Gives the room of the rule placed last back (a rule that could not be made); returns rc.  Kernels of the
+  // rule may have been launched on s: the room is free when they have finished.
+  int unplace_rule(dfrg_qp *qp, const Rule &r, int rc, hipStream_t s)
   {
+    (void)hipStreamSynchronize(s);
     qp->slab_used = (size_t)((char *)r.d_x - qp->slabs.back());
     return rc;
   }
@@ -573,7 +575,7 @@ int dfrg_qp_gl(dfrg_qp *qp, int order, int fp32, const void **d_x, const void **
     hipStream_t s = resolve_stream(nullptr);
     int rc = dfrg_gl_generate(order, r.d_x, r.d_w, s);
     if (rc == DFRG_OK) rc = finish_rule(r, s);
-    if (rc != DFRG_OK) return unplace_rule(qp, r, rc);
+    if (rc != DFRG_OK) return unplace_rule(qp, r, rc, s);
     it = qp->gl.emplace(order, std::move(r)).first;
   }
   hand_out(it->second, fp32, d_x, d_w, h_x, h_w);
@@ -601,7 +603,7 @@ int dfrg_qp_matsubara(dfrg_qp *qp, double T, double E, int fp32, int *size, doub
     int rc = enqueue_matsubara(tit->first, E, 2, qp->min_matsubara_size, 128, qp->vacuum_quad_size,
                                qp->add_matsubara_size, r.d_x, r.d_w, cap, &r.size, &r.T_rule, s);
     if (rc == DFRG_OK) rc = finish_rule(r, s);
-    if (rc != DFRG_OK) return unplace_rule(qp, r, rc);
+    if (rc != DFRG_OK) return unplace_rule(qp, r, rc, s);
     eit = emap.emplace(E, std::move(r)).first;
   }
   if (size) *size = eit->second.size;
