@@ -403,8 +403,14 @@ namespace
       set_error("flow graph capture failed: %s", hipGetErrorString(e));
       return DFRG_ERR_HIP;
     }
+    e = hipGraphInstantiate(&fs->graph_exec[g], gr, nullptr, nullptr, 0);
+    if (e != hipSuccess) {
+      (void)hipGraphDestroy(gr);
+      fs->graph_exec[g] = nullptr;
+      set_error("flow graph instantiation failed: %s", hipGetErrorString(e));
+      return DFRG_ERR_HIP;
+    }
     fs->graph[g] = gr;
-    DFRG_HIP(hipGraphInstantiate(&fs->graph_exec[g], gr, nullptr, nullptr, 0));
     *exec = fs->graph_exec[g];
     return DFRG_OK;
   }

@@ -54,3 +54,23 @@ assert "L" in log and "M" in log and "S" in log[log.rindex("L"):], log
 fake.fake_fail(0, 0)
 assert {call} == 0
 """)
+
+
+def test_flow_graph_that_cannot_be_instantiated_is_destroyed(run):
+    run("""
+fs, fid = C.c_void_p(), C.c_longlong()
+D.check(L.dfrg_fs_create(C.byref(fs), qp, 1 << 20, 4, 64, 100, 0.3, 10))
+desc = D.FlowDesc(64, 4.0, 0.2, 0.0, 4.0, 0.2, 1.0)
+D.check(L.dfrg_fs_submit(fs, C.byref(desc), C.byref(fid)))
+fake.fake_clear()
+fake.fake_fail(0, 1)
+for _ in range(3):
+    assert L.dfrg_fs_progress(fs, None, None, None) != 0
+log = fake.fake_log().decode()
+assert log.count("C") == log.count("D") == 3, log
+fake.fake_fail(0, 0)
+D.check(L.dfrg_fs_progress(fs, None, None, None))
+D.check(L.dfrg_fs_destroy(fs))
+log = fake.fake_log().decode()
+assert log.count("C") == log.count("D"), log
+""")
