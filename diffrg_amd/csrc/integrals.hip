@@ -563,19 +563,23 @@ namespace
     return acc;
   }
 
-  // MODE DFRG_FP64 holds both FP64 forms (per tile); kSeededOnly, for batches whose integrals all
-  // admit the seeded form, only that one, with its register budget (the library sequences of the
-  // general form need 168 VGPRs).
-  constexpr int kSeededOnly = 2;
+  // The FP64 kernels: MODE DFRG_FP64 holds the general form, kSeeded the seeded one and kBothForms both, chosen
+  // per tile.  A batch whose integrals all take one form runs that form's kernel, with its register budget
+  // (about 120 VGPRs; 168 with both, three waves per SIMD instead of four): 512 integrals of {64, 32, 32}
+  // nodes in the general form take 204 us there against 210.5 in the kernel with both.  A mixed batch keeps one
+  // launch, as two would run one form's tiles after the other's last wave: one integral in the general
+  // form among 512 takes 75 us, against 61 without it and 21 for it alone.
+  constexpr int kSeeded = 2, kBothForms = 3;
   template <int MODE, int BLOCK, int UNROLL> __global__ __launch_bounds__(BLOCK) void se_kernel(SEArgs A)
   {
-    constexpr bool F64 = MODE != DFRG_MIXED, GENERAL = MODE == DFRG_FP64;
+    constexpr bool F64 = MODE != DFRG_MIXED, GENERAL = MODE == DFRG_FP64 || MODE == kBothForms;
+    constexpr bool SEEDED = MODE == kSeeded || MODE == kBothForms;
     __shared__ double s_tab64[GENERAL ? kMaxTab : 1];
     __shared__ SECellY s_tabA[F64 ? 1 : kMaxTab];
-    __shared__ SECellZ s_tabB[kMaxTab];
-    __shared__ double2 s_log[F64 ? dev::kLogTab : 1];
+    __shared__ SECellZ s_tabB[SEEDED || !F64 ? kMaxTab : 1];
+    __shared__ double2 s_log[SEEDED ? dev::kLogTab : 1];
     __shared__ double s_exp2[F64 ? 1 : 64]; // 2^(j/64)
-    __shared__ double s_exp2k[64];          // k^2 2^(j/64)
+    __shared__ double s_exp2k[SEEDED || !F64 ? 64 : 1]; // k^2 2^(j/64)
     __shared__ double2 s_ang[kMaxAng]; // (cos1, 2 w1 sqrt(1 - cos1^2))
     __shared__ double s_w2[kMaxAng];   // 2 w2
     __shared__ double s_qs[kMaxQ], s_qc[kMaxQ], s_qt[kMaxQ];
@@ -590,7 +594,7 @@ namespace
         s_exp2[j] = exp2(j * (1.0 / 64.0));
         s_exp2k[j] = A.k * A.k * s_exp2[j];
       }
-    } else if ((int)threadIdx.x >= BLOCK - 64) {
+    } else if (SEEDED && (int)threadIdx.x >= BLOCK - 64) {
       const int j = (int)threadIdx.x - (BLOCK - 64);
       s_exp2k[j] = A.k * A.k * ((const double *)(A.logtab + dev::kLogTab))[j];
     }
@@ -621,7 +625,7 @@ namespace
       // one round of independent loads: table and angular terms (when the integral changes) and
       // the radial nodes of this tile
       if (i != cur) {
-        if (F64 && (!GENERAL || T.seeded)) {
+        if (SEEDED && (!GENERAL || T.seeded)) {
           for (int j = threadIdx.x; j < T.ntab; j += BLOCK) s_tabB[j] = A.tabB[T.tab_off + j];
           for (int j = threadIdx.x; j < dev::kLogTab; j += BLOCK) {
             const double2 l = A.logtab[j];
@@ -653,7 +657,7 @@ namespace
       }
       __syncthreads();
       SESeeded S; // the seeded FP64 form's constants (unused otherwise)
-      if (F64) {
+      if (SEEDED) {
         S.tabB = s_tabB;
         S.lg = s_log;
         S.exp2k = s_exp2k;
@@ -672,7 +676,7 @@ namespace
         const double2 qw = s_qw[j];
         const double q = qw.x, q2 = q * q;
         double qt;
-        if (F64 && (!GENERAL || T.seeded)) {
+        if (SEEDED && (!GENERAL || T.seeded)) {
           const double R = S.R(q2), Gq = dev::rcp_f64(fma(S.Z(q), q2, R));
           const double el = A.pref * (q2 * 0.5 * k2);
           qt = el * qw.y * (2.0 * R * (1.0 + q2 / k2)) * Gq * Gq;
@@ -701,7 +705,7 @@ namespace
       __syncthreads();
 
       double acc;
-      if (F64 && (!GENERAL || T.seeded)) { // tile-uniform
+      if (SEEDED && (!GENERAL || T.seeded)) { // tile-uniform
         acc = se_tile_sum<BLOCK, UNROLL>(S, T.na, T.l2na, T.nqt, s_ang, s_w2, s_qs, s_qc, s_qt);
       } else if (GENERAL) {
         const auto g = [&](double pq2) { return se_G_fp64(s_tab64, T.ntab, T.c, T.inv_b, T.scale, k2, pq2); };
@@ -810,7 +814,7 @@ struct dfrg_se_batch {
   int block = 256, tile_evals = 8192, grid = 0, n_tiles = 0;
   std::vector<int> narrow; // per integral: the mixed path may use se_G_mixed<true>
   std::vector<int> seeded; // per integral: the FP64 path may use SESeeded
-  bool all_seeded = false;
+  int n_seeded = 0;
   int uniform_tiles = 0;    // every tile has the same evaluation count
   int shared_layout = 0;    // every tile record follows from proto and its index (SEArgs::shared)
   int tiles_per_int = 0;
@@ -960,11 +964,13 @@ namespace
       a.queue = scr->queue;
     }
     const int grid = b->grid > 0 ? std::min(b->grid, b->n_tiles) : b->n_tiles;
-    hipError_t e = mode == DFRG_FP64
-                       ? (b->all_seeded ? (se_unroll(b) == 2 ? launch_se<kSeededOnly, 2>(b->block, grid, s, a) : launch_se<kSeededOnly, 1>(b->block, grid, s, a))
-                                        : launch_se<DFRG_FP64, 1>(b->block, grid, s, a))
-                   : se_unroll(b) == 2 ? launch_se<DFRG_MIXED, 2>(b->block, grid, s, a)
-                                       : launch_se<DFRG_MIXED, 1>(b->block, grid, s, a);
+    const bool two = se_unroll(b) == 2;
+    hipError_t e = mode == DFRG_MIXED ? (two ? launch_se<DFRG_MIXED, 2>(b->block, grid, s, a)
+                                             : launch_se<DFRG_MIXED, 1>(b->block, grid, s, a))
+                   : b->n_seeded == b->n_int ? (two ? launch_se<kSeeded, 2>(b->block, grid, s, a)
+                                                    : launch_se<kSeeded, 1>(b->block, grid, s, a))
+                   : b->n_seeded == 0 ? launch_se<DFRG_FP64, 1>(b->block, grid, s, a)
+                                      : launch_se<kBothForms, 1>(b->block, grid, s, a);
     if (e != hipSuccess) {
       set_error("launch of se_kernel failed: %s", hipGetErrorString(e));
       return DFRG_ERR_HIP;
@@ -1172,7 +1178,7 @@ int dfrg_se_batch_create(dfrg_se_batch **out, dfrg_qp *qp, int n_int, const doub
     for (int j = 0; ok && j < tab_n[i]; ++j) ok = std::fabs(tables[tab_off[i] + j]) < 0x1p1000;
     b->seeded[i] = ok;
   }
-  b->all_seeded = std::all_of(b->seeded.begin(), b->seeded.end(), [](int v) { return v != 0; });
+  b->n_seeded = std::accumulate(b->seeded.begin(), b->seeded.end(), 0);
   // log and exp tables of the seeded form
   std::vector<double> logtab(2 * dev::kLogTab + 64);
   for (int j = 0; j < dev::kLogTab; ++j) {
