@@ -108,7 +108,11 @@ namespace
   }
 
   constexpr int kThGroup = 8, kThBlock = 1024;
-  constexpr int kThWaveMax = 4096; // largest batch of threshold_wave_kernel: 2.8 us against 3.5 there, 3.6 against 3.6 at 8,192
+  // Largest batch of threshold_wave_kernel.  Up to 64 nodes 2.8 us against 3.5 there, 3.6 against 3.6 at 8,192; up to
+  // 256 nodes 5.4 against 5.5 at 4,097 and 6.7 against 5.6 at 6,000.  Past the 256 nodes whose terms a block
+  // keeps, where a group's wave forms them again: of 300, 600 and 1,024 nodes 7.8, 13.3 and 20.3 us against
+  // 9.3, 16.3 and 24.1 at 6,000, 9.5, 16.9 and 25.8 against 9.4, 16.2 and 24.2 at 8,192.
+  constexpr int th_wave_max(int nx) { return nx <= 256 ? 4096 : 7680; }
   template <int MODE, int R>
   __global__ __launch_bounds__(kThBlock) void threshold_kernel(int d, const double *__restrict__ m2, int n_int,
                                                                const double *__restrict__ x,
@@ -1001,7 +1005,7 @@ int dfrg_threshold_batch(int d, const double *d_m2, int n_int, const double *d_x
   DFRG_CHECK_ARG(d_m2 && d_x && d_w && d_out, "NULL device pointer");
   const double pref = S_d_host(d) / std::pow(2.0 * kPi, d);
   hipStream_t s = resolve_stream(stream);
-  if (n_int <= kThWaveMax) {
+  if (n_int <= th_wave_max(nx)) {
     const auto kernel =
         mode == DFRG_FP64 ? threshold_wave_kernel<DFRG_FP64> : threshold_wave_kernel<DFRG_MIXED>;
     hipLaunchKernelGGL(kernel, dim3((n_int + 3) / 4), dim3(256), 0, s, d, d_m2, n_int, d_x, d_w, nx, x_extent, k, pref,

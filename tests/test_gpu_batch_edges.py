@@ -34,6 +34,27 @@ def test_threshold_sizes(gpu, qp, nx, n, k, d):
         assert np.abs(got[:n] / ref - 1).max() <= TOL
 
 
+# both sides of the batch size at which the kernel changes; the first integrals of a larger batch are the same
+# bits as alone, in either kernel
+@pytest.mark.parametrize("nx,limit", [(7, 4096), (64, 4096), (100, 4096), (256, 4096), (257, 7680), (600, 7680),
+                                      (1024, 7680)])
+def test_threshold_bits_across_the_kernels(gpu, qp, nx, limit):
+    m2 = np.random.default_rng(nx).uniform(-0.9, 4.0, limit + 13)
+    x, w = qp.get_points(nx), qp.get_weights(nx)
+    ref = O.c0_threshold(m2, x, w, 20.0, 1.0, 1.0, 4)
+    d_x, d_w = (gpu.DeviceArray.from_host(a) for a in (x, w))
+    for mode in (gpu.FP64, gpu.MIXED):
+        res = []
+        for n in (5, limit, limit + 1, limit + 13):
+            print(f"[case] threshold n={n} nx={nx} mode={mode}", flush=True)
+            out = gpu.DeviceArray(n)
+            gpu.threshold_batch(gpu.DeviceArray.from_host(m2[:n]), d_x, d_w, out, 20.0, 1.0, mode, 4)
+            res.append(out.to_host())
+            assert np.abs(res[-1] / ref[:n] - 1).max() <= TOL
+        for r in res[:-1]:
+            assert np.array_equal(r, res[-1][:len(r)])
+
+
 def test_threshold_special_masses(gpu, qp):
     # infinite masses give 0, NaN gives NaN; a neighbour in the same group of eight is not touched
     x, w = qp.get_points(33), qp.get_weights(33)
