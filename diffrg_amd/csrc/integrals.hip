@@ -87,7 +87,9 @@ namespace
     return fma(F * G, G, v);
   }
 
-  // Small batches, one wave per integral: nothing to share, and the launch bounds them.
+  // Small batches, one wave per integral: nothing to share, and the launch bounds them.  (blockDim.x, not a
+  // constant: its load takes the second line of the kernel's arguments beside the first's, where the rest
+  // would wait for the exit test in between; 64 integrals 2.36 against 2.52 us.)
   template <int MODE>
   __global__ __launch_bounds__(256) void threshold_wave_kernel(int d, const double *__restrict__ m2, int n_int,
                                                                const double *__restrict__ x,
@@ -95,7 +97,7 @@ namespace
                                                                double k, double pref, double *__restrict__ out)
   {
     const int lane = threadIdx.x & 63;
-    const int integral = (blockIdx.x * 256 + threadIdx.x) >> 6;
+    const int integral = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     if (integral >= n_int) return; // whole wave exits together
     const double m = m2[integral];
     double v = 0.0;
