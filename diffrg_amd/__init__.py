@@ -93,6 +93,7 @@ SIGNATURES = {
     "dfrg_se_batch_graph_launch": [_vp, C.c_int, _vp, C.c_int, _vp],
     "dfrg_se_batch_evals": [_vp, C.POINTER(C.c_ulonglong)],
     "dfrg_se_batch_variants": [_vp, C.c_int, _ip],
+    "dfrg_se_batch_seeded": [_vp, _ip],
     "dfrg_se_batch_unroll": [_vp, _ip],
     "dfrg_se_batch_run_noalloc": [_vp, C.c_int, _vp, _vp],
     "dfrg_ft_set_block": [C.c_int],
@@ -492,9 +493,16 @@ class SEBatch:
         check(lib().dfrg_se_batch_variants(self.ptr, mode, v.ctypes.data_as(C.POINTER(C.c_int))))
         return v
 
+    @property
+    def seeded(self) -> np.ndarray:
+        """Per integral: an FP64 run evaluates it in the seeded form (False: by the math library)."""
+        v = np.empty(self.n, dtype=np.int32)
+        check(lib().dfrg_se_batch_seeded(self.ptr, v.ctypes.data_as(C.POINTER(C.c_int))))
+        return v.astype(bool)
+
     def unroll(self, mode: int) -> int:
         """Radial unroll of the paired evaluation loop a run in `mode` uses at the current shape."""
-        if mode == FP64:
+        if mode == FP64 and not self.seeded.all():
             return 1
         u = C.c_int()
         check(lib().dfrg_se_batch_unroll(self.ptr, C.byref(u)))

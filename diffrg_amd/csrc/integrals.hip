@@ -1321,6 +1321,13 @@ int dfrg_se_batch_variants(dfrg_se_batch *b, int mode, int *variant)
   return DFRG_OK;
 }
 
+int dfrg_se_batch_seeded(dfrg_se_batch *b, int *seeded)
+{
+  DFRG_CHECK_ARG(b && seeded, "NULL argument");
+  std::copy(b->seeded.begin(), b->seeded.end(), seeded);
+  return DFRG_OK;
+}
+
 int dfrg_se_batch_unroll(dfrg_se_batch *b, int *unroll)
 {
   DFRG_CHECK_ARG(b && unroll, "NULL argument");

@@ -192,15 +192,21 @@ int dfrg_se_batch_autotune(dfrg_se_batch *b, int mode, int reps, const char *cac
 int dfrg_se_batch_graph_launch(dfrg_se_batch *b, int mode, double *d_out, int launches, void *stream);
 /* Evaluations (integrand calls) performed by one run of the batch. */
 int dfrg_se_batch_evals(dfrg_se_batch *b, unsigned long long *evals);
-/* Integrand form a run in `mode` uses for each integral (variant[0 .. n_int-1]): 0 FP64; 1 mixed;
+/* Integrand form a run in `mode` uses for each integral (variant[0 .. n_int-1]): 0 FP64 (which of its
+ * two: dfrg_se_batch_seeded); 1 mixed;
  * 2 mixed for an integral whose table starts at >= 1e-30 and whose |p - q|^2 64 log2(e)/k^2
  * stays below 2^30, which rounds the exponent with one FMA and drops a guard (within the mixed
  * tolerance of form 1).  The choice depends on the integral alone, not on the batch. */
 int dfrg_se_batch_variants(dfrg_se_batch *b, int mode, int *variant);
-/* Radial unroll of the mixed path's paired evaluation loop at the current shape: 2 (two radial
- * nodes per step) when the launch puts at most 16 waves on a CU, else 1.  The plain path's general
- * form always uses 1; its seeded form follows the same rule as the mixed path.  Results do not
- * depend on it. */
+/* seeded[i] = 1 where a DFRG_FP64 run evaluates integral i in the seeded form (tables for log and exp,
+ * hardware reciprocal estimates refined in FP64), 0 where it calls the math library: a coordinate map
+ * of bias below 2, a table that starts at 0, or a table with infinite values.  The choice depends on
+ * the integral alone, not on the batch. */
+int dfrg_se_batch_seeded(dfrg_se_batch *b, int *seeded);
+/* Radial unroll of the paired evaluation loop at the current shape, of the mixed path and of the plain
+ * path when every integral takes the seeded form: 2 (two radial nodes per step) when the launch puts at
+ * most 16 waves on a CU, else 1.  The plain path's other kernels always use 1.  Results do not depend on
+ * it. */
 int dfrg_se_batch_unroll(dfrg_se_batch *b, int *unroll);
 
 /* dfrg_se_batch_run without any allocation.  No counterpart in the reference: it is for callers

@@ -74,6 +74,22 @@ def test_general_fp64_beside_seeded(gpu, qp):
         assert one.to_host()[0] == got[i]
 
 
+@pytest.mark.gpu
+def test_seeded_and_unroll_queries(gpu, qp):
+    z = np.linspace(1.0, 1.5, 48)
+    start = np.array([1e-3, 1e-3, 0.0, 1e-3])
+    bias = np.array([6.0, 1.0, 6.0, 2.0])
+    tables = [z.copy() for _ in bias]
+    b = gpu.SEBatch(qp, np.ones(4), 32, 16, tables, start, 40.0, bias)
+    assert list(b.seeded) == [True, False, False, True]
+    # the kernel that holds both FP64 forms takes one radial node per step
+    assert b.unroll(gpu.FP64) == 1 and b.unroll(gpu.MIXED) == 2
+    thin = gpu.SEBatch(qp, np.ones(4), 32, 16, tables, 1e-3, 40.0, 6.0)
+    assert thin.seeded.all() and thin.unroll(gpu.FP64) == thin.unroll(gpu.MIXED) == 2
+    thick = gpu.SEBatch(qp, np.ones(300), 64, 64, [z] * 300, 1e-3, 40.0, 6.0)
+    assert thick.unroll(gpu.FP64) == thick.unroll(gpu.MIXED) == 1
+
+
 @pytest.mark.skipif(not os.path.exists(I.B.HIPCC), reason="hipcc not found")
 def test_seeded_loop_counts_match_bench():
     import bench
