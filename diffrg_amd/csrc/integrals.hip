@@ -314,7 +314,6 @@ namespace
       __syncthreads();
       for (int n = lane; n < nm; n += 64) {
         const double wn = A.mx[off + n], wgt = A.mw[off + n], dp = wn + p0, dm = -wn + p0;
-#pragma unroll 2
         for (int j = wv; j < nx; j += NW) {
           const double rd = s_rd[j], a2 = s_a2[j];
           const double g1 = 1.0 / (wn * wn + s_a1[j]), gp = 1.0 / (dp * dp + a2), gm = 1.0 / (dm * dm + a2);
