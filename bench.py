@@ -42,18 +42,23 @@ GRAPH_SETS = 10  # call sets per hipGraph launch
 # loops of se_kernel<MODE, BLOCK, UNROLL>, counted from the gfx950 assembly of
 # csrc/integrals.hip by `python -m diffrg_amd.isa_count`: "pairs" when a lane owns two angular
 # pairs (na^2 >= 2 BLOCK), "pairs2" the same loop taking two radial nodes per step (the mixed
-# unroll 2, SEBatch.unroll(MIXED), which the seeded FP64 form shares), "single" when a lane owns one pair and two radial nodes per
+# unroll 2, SEBatch.unroll), "single" when a lane owns one pair and two radial nodes per
 # iteration.  tests/test_isa_counts.py checks these figures against the current source.
-# Keyed by the integrand form (SEBatch.variants): 0 FP64, 1 mixed, 2 mixed on an integral that
-# admits the narrow exponent rounding.
-# FP64 runs the seeded form ("seeded") on integrals whose coordinates and tables admit it, as those of
-# every workload here do, and the library-call form 0 on the others.
+# Keyed by the integrand form (se_form): 0 FP64 by library calls, "seeded" FP64 by tables and hardware
+# estimates, 1 mixed, 2 mixed on an integral that admits the narrow exponent rounding.
 SE_OPS = {0: {"pairs": (223.5, 203.0), "single": (223.5, 205.0)},
           "seeded": {"pairs": (63.5, 50.0), "pairs2": (63.25, 49.0), "single": (63.5, 52.0)},
           1: {"pairs": (46.0, 44.0), "pairs2": (46.0, 43.5), "single": (46.0, 46.0)},
           2: {"pairs": (46.0, 42.0), "pairs2": (46.0, 41.5), "single": (46.0, 44.0)}}
 # (form, block, loop) whose schedule differs from the others
 SE_OPS_BLOCK = {}
+
+# The same of the other kernels whose loops do other work than the frozen weights below were counted on: per
+# radial node (threshold, one wave per integral), frequency pair (finite-T) and node of both threshold
+# integrals (flow step, eight lanes per integral).  tests/test_isa_counts.py checks them.
+EXECUTED = {"C0_threshold": {"fp64": {"flop": 91.0, "valu": 80.0}, "mixed": {"flop": 88.0, "valu": 80.0}},
+            "C2_finite_T": {"fp64": {"flop": 18.0, "valu": 14.75}, "mixed": {"flop": 18.0, "valu": 14.75}},
+            "C4_flow_node": {"fp64": {"flop": 90.0, "valu": 83.0}}}
 
 
 BASELINE_NOTES = "BASELINE.md"
@@ -68,6 +73,12 @@ def frozen_weights():
 
 
 FROZEN = frozen_weights()
+
+
+def weights(workload, mode):
+    """FLOP and VALU per evaluation of a workload's kernel: the counts of the current loop where it differs from the
+    frozen one, so that a fraction of peak is of executed work."""
+    return EXECUTED.get(workload, FROZEN[workload])[mode]
 
 
 def ceiling(w):
@@ -90,14 +101,22 @@ def se_ops(variant, na, block, unroll=1):
 
 def se_variant(b, mode):
     """The integrand form of a batch whose integrals all use the same one."""
-    v = np.unique(b.variants(mode))
+    v = set(se_form(b, mode))
     assert len(v) == 1, v
-    return se_form(v[0])
+    return v.pop()
 
 
-def se_form(variant):
-    """Key of SE_OPS for SEBatch.variants' value on the integrals of these workloads."""
-    return "seeded" if variant == 0 else int(variant)
+def se_form(b, mode):
+    """Keys of SE_OPS for the integrals of a batch."""
+    return ["seeded" if v == 0 and s else int(v) for v, s in zip(b.variants(mode), b.seeded)]
+
+
+def se_weights(workload, variant, na, block, unroll):
+    """weights() of the self-energy loops: the mixed forms at their frozen weights, the FP64 ones as counted."""
+    if variant in (1, 2):
+        return FROZEN[workload]["mixed"]
+    flop, valu = se_ops(variant, na, block, unroll)
+    return {"flop": flop, "valu": valu}
 
 
 def valu_issue_frac(valu_per_eval, evals, seconds):
@@ -299,7 +318,7 @@ def selfenergy(D, qp, args):
                 err = max(err, rel_err(o.to_host(), ref))
         ms = min(ms_eager, ms_graph)
         res[name] = {"ms": ms, "ms_eager": ms_eager, "ms_graph": ms_graph, "ms_streams": ms_streams, "shape": shape,
-                     "err": err, "launch": "hipGraph" if ms_graph < ms_eager else "eager", "unroll": b.unroll(D.MIXED)}
+                     "err": err, "launch": "hipGraph" if ms_graph < ms_eager else "eager", "unroll": b.unroll(mode)}
         log(f"selfenergy {name}: eager {ms_eager * 1e3:.1f} us, graph {ms_graph * 1e3:.1f} us, "
             f"{N_STREAMS} streams {ms_streams * 1e3:.1f} us per call set, "
             f"err {err:.2e}, shape {shape}")
@@ -316,8 +335,9 @@ def selfenergy(D, qp, args):
     for mode, name in ((D.FP64, "fp64"), (D.MIXED, "mixed")):
         shape = bb.autotune(mode, reps=3)
         ms, _ = time_steps(D, lambda: bb.run(outb, mode), max(1, args.steps // BATCH), max(1, args.warmup // BATCH))
-        va = se_ops(se_variant(bb, mode), c["na"], shape["block"], bb.unroll(D.MIXED))[1]
-        fl = FROZEN["C1_selfenergy"][name]["flop"]
+        form, unroll = se_variant(bb, mode), bb.unroll(mode)
+        va = se_ops(form, c["na"], shape["block"], unroll)[1]
+        fl = se_weights("C1_selfenergy", form, c["na"], shape["block"], unroll)["flop"]
         res[name][f"batched_x{BATCH}"] = {
             "integrals_per_s": nb / (ms * 1e-3), "us_per_launch": ms * 1e3, "shape": shape,
             "max_rel_err": rel_err(outb.to_host(), refb),
@@ -342,7 +362,7 @@ def threshold(D, qp, args):
         run = lambda: D.threshold_batch(d_m2, d_x, d_w, out, c["x_extent"], c["k"], mode, c["d"])
         ms_e, ms_g = eager_and_graph(D, run, args)
         ms = min(ms_e, ms_g)
-        wt = FROZEN["C0_threshold"][name]
+        wt = weights("C0_threshold", name)
         r[name] = {"integrals_per_s": len(c["m2"]) / (ms * 1e-3), "us_per_step": ms * 1e3,
                    "us_eager": ms_e * 1e3, "us_graph": ms_g * 1e3, "launch": "hipGraph" if ms_g < ms_e else "eager",
                    "max_rel_err": rel_err(out.to_host(), ref),
@@ -391,7 +411,7 @@ def finite_T(D, qp, args):
         ms = min(ms_e, ms_g)
         got = out.to_host()
         err = np.abs(got - ref) / np.abs(ref)
-        wt = FROZEN["C2_finite_T"][name]
+        wt = weights("C2_finite_T", name)
         pairs = int(sum(c["nx"] * len(c["rules"][t][0]) for t in c["T"]))
         r[name] = {"integrals_per_s": len(c["T"]) / (ms * 1e-3), "evals_per_s": evals / (ms * 1e-3),
                    "us_per_step": ms * 1e3, "us_eager": ms_e * 1e3, "us_graph": ms_g * 1e3,
@@ -449,15 +469,16 @@ def uneven(D, qp, args):
         shape = b.autotune(mode, reps=2, cache_path=None)
         ms, _ = time_steps(D, lambda: b.graph_launch(out, mode, launches=per_graph), steps, 2)
         ms /= per_graph
-        wt = FROZEN["C3_uneven"][name]
+        # integrals of the four angular orders run different loops: totals over the batch
+        work = [(int(q) * int(a) ** 2, int(a), v) for q, a, v in zip(c["nq"], c["na"], se_form(b, mode))]
+        unroll = b.unroll(mode)
+        valu = sum(e * se_ops(v, a, shape["block"], unroll)[1] for e, a, v in work)
+        wts = [(e, se_weights("C3_uneven", v, a, shape["block"], unroll)) for e, a, v in work]
+        tot = {key: sum(e * w[key] for e, w in wts) for key in ("flop", "valu")}
         r[name] = {"integrals_per_s": n / (ms * 1e-3), "evals_per_s": b.evals / (ms * 1e-3), "ms_per_batch": ms,
                    "max_rel_err": rel_err(out.to_host(), ref), "shape": shape,
-                   "roofline_frac": wt["flop"] * b.evals / (ms * 1e-3) / PEAK_FP64_VALU, "ceiling": ceiling(wt),
-                   "valu_issue_frac": sum(int(q) * int(a) ** 2 * se_ops(se_form(v), int(a), shape["block"],
-                                                                          b.unroll(D.MIXED))[1]
-                                          for q, a, v in zip(c["nq"], c["na"], b.variants(mode)))
-                                      / 64 / (ms * 1e-3)
-                                      / PEAK_VALU_WAVE_INSTR}
+                   "roofline_frac": tot["flop"] / (ms * 1e-3) / PEAK_FP64_VALU, "ceiling": ceiling(tot),
+                   "valu_issue_frac": valu / 64 / (ms * 1e-3) / PEAK_VALU_WAVE_INSTR}
         log(f"uneven {name}: {ms:.3f} ms/batch, err {r[name]['max_rel_err']:.2e}, shape {shape}")
     r["mixed_over_plain"] = r["mixed"]["integrals_per_s"] / r["fp64"]["integrals_per_s"]
     r["cpu_integrals_per_s"] = n / t_cpu
@@ -542,9 +563,9 @@ def _flow_sample(reqs, m, seed):
 def flow_step_roofline(tm, nx=64):
     """flow_step_kernel over the steady-state run, from the server's HIP events around each graph
     launch (25 step launches and the base-step node per graph, so the gaps between the launches
-    inside a graph count as kernel time): frozen FLOP per node of both threshold integrals x 64
+    inside a graph count as kernel time): FLOP per node of both threshold integrals x 64
     nodes x 4 RK stages per grid-point step."""
-    wt = FROZEN["C4_flow_node"]["fp64"]
+    wt = weights("C4_flow_node", "fp64")
     node_evals = tm["point_steps"] * 4 * nx
     achieved = wt["flop"] * node_evals / tm["device_s"] if tm["device_s"] > 0 else 0.0
     return {"graph_launches": tm["launches"], "device_s": tm["device_s"], "point_steps": tm["point_steps"],
@@ -680,9 +701,10 @@ def main():
     }
     na = se["na"]
     v1 = se["variant"][1]
-    # FLOP per evaluation: the frozen weights; VALU per evaluation: the current
-    # assembly of the loop that ran (for the issue fraction)
-    w1, w0 = FROZEN["C1_selfenergy"]["mixed"], FROZEN["C1_selfenergy"]["fp64"]
+    # FLOP per evaluation: the frozen weights of the mixed form, the loop that ran in FP64; VALU per
+    # evaluation: the current assembly of the loop that ran (for the issue fraction)
+    w1 = FROZEN["C1_selfenergy"]["mixed"]
+    w0 = se_weights("C1_selfenergy", se["variant"][0], na, fp["shape"]["block"], fp["unroll"])
     fl1, fl0 = w1["flop"], w0["flop"]
     va1 = se_ops(v1, na, mx["shape"]["block"], mx["unroll"])[1]
     va0 = se_ops(se["variant"][0], na, fp["shape"]["block"], fp["unroll"])[1]
@@ -696,7 +718,9 @@ def main():
                        "loop": se_loop(na, mx["shape"]["block"], mx["unroll"]),
                        "evals_per_launch": evals,
                        "valu_issue_frac": valu_issue_frac(va1, evals, mx["ms"] * 1e-3),
-                       "plain_fp64": {"flop_per_eval": fl0, "valu_per_eval": va0, "ceiling": ceiling(w0),
+                       "plain_fp64": {"integrand_form": {0: "library", "seeded": "seeded"}[se["variant"][0]],
+                                      "flop_per_eval": fl0, "flop_per_eval_source": "the loop's assembly",
+                                      "valu_per_eval": va0, "ceiling": ceiling(w0),
                                       "loop": se_loop(na, fp["shape"]["block"], fp["unroll"]),
                                       "achieved": fl0 * evals / (fp["ms"] * 1e-3) / 1e12,
                                       "frac": fl0 * evals / (fp["ms"] * 1e-3) / PEAK_FP64_VALU,

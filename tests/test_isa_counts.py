@@ -46,6 +46,27 @@ def test_se_kernel_counts_match_bench():
                 assert bench.se_ops(form, na, block, unroll) == per_eval, (name, form, kind, c)
 
 
+@pytest.mark.skipif(not os.path.exists(I.B.HIPCC), reason="hipcc not found")
+def test_executed_counts_match_bench():
+    csrc = os.path.join(ROOT, "diffrg_amd", "csrc")
+    with tempfile.TemporaryDirectory() as d:
+        batch = I.inner_loops(I.compile_asm(os.path.join(csrc, "integrals.hip"), d))
+        flow = I.inner_loops(I.compile_asm(os.path.join(csrc, "flow.hip"), d))
+    per = lambda c, n: {"flop": c["flop"] / n, "valu": c["valu"] / n}
+    for mode, name in ((0, "fp64"), (1, "mixed")):
+        body = [c for n, c in batch if f"threshold_wave_kernelILi{mode}E" in n]
+        assert [per(c, 1) for c in body] == [bench.EXECUTED["C0_threshold"][name]]
+    for block in (64, 128, 256, 512):
+        # one reciprocal per pair, four pairs per step: the uniform loop reads the radial terms of two nodes at a time
+        body = [c for n, c in batch if f"ft_kernelILi{block}E" in n and c["trans"] == 4]
+        c = min(body, key=lambda c: c["valu"])
+        assert per(c, 4) == bench.EXECUTED["C2_finite_T"]["fp64"] == bench.EXECUTED["C2_finite_T"]["mixed"]
+    # two seeds per evaluation; the loop of eight lanes per integral adds a second group of four to the first
+    body = [c for n, c in flow if "flow_step_kernel" in n and c["trans"] == 8]
+    c = max(body, key=lambda c: c["valu"])
+    assert per(c, 2) == bench.EXECUTED["C4_flow_node"]["fp64"]
+
+
 def test_se_loop_choice():
     # se_tile_sum: a lane owns two angular pairs when na^2 >= 2 * BLOCK
     assert bench.se_loop(32, 256) == "pairs" and bench.se_loop(32, 512) == "pairs"
