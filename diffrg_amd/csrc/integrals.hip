@@ -162,7 +162,8 @@ namespace
           }
       }
       const double sum = dev::wave_sum8(v);
-      const int u = 4 * ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1) + (lane >> 5); // the vector this lane's sum belongs to
+      // the vector this lane's sum belongs to
+      const int u = 4 * ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1) + (lane >> 5);
       if ((lane & 7) == 0 && u < left) out[i0 + u] = sum;
     }
   }
@@ -197,8 +198,10 @@ namespace
   // General: three IEEE divisions per pair, as in the reference.  For integrals beyond those limits, whose
   // accumulator becomes NaN, and for those whose fast sum is not finite (a vanishing denominator makes
   // the reciprocal NaN): a sum that is not finite sends its block through this form.
-  // (An FP32 seed in mixed mode, at 24.0 us against 25.8 for 8,191 integrals of 48 nodes, lost terms without a
-  // sign where k is below 1e-5 of a mass: the product of three denominators leaves the FP32 range.)
+  // 16,384 integrals of 48 nodes 28.5 -> 27.6 us against the reciprocal of any product, with its fix-up of special
+  // values (three divisions: 80).  An FP32 seed in mixed mode would take 26.5, but lost terms without a sign
+  // where k is below 1e-5 of a mass: the product of three denominators leaves the FP32 range.  4,096 integrals
+  // of infinite mass, general form: 31.7 us.
   constexpr double kFtLimit = 0x1p246;
   template <int BLOCK> __global__ __launch_bounds__(BLOCK) void ft_kernel(FTArgs A)
   {

@@ -308,8 +308,8 @@ namespace dfrg
     // the entry (1/c_j rounded, -log of that value), r = m/c_j - 1 exact to one rounding, |r| <= 2^-8, and
     // log1p(r) = r + r^2 P(r) with P of degree 3 (Chebyshev interpolation; remainder 7.5e-17).  The
     // entry's second value and ln2 come multiplied by `scale`, so the result is scale log(w); absolute
-    // error about one rounding of the largest term.  w must be positive and normal; a NaN w gives a
-    // large finite value.
+    // error about one rounding of the largest term.  w must be positive and normal; a NaN w gives NaN, and the
+    // caller's clamp has to drop it (fmin and fmax do).
     constexpr int kLogTab = 128;
     __device__ __forceinline__ double log_tab(double w, const double2 *tab, double scale, double scale_ln2)
     {
